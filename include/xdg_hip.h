@@ -122,7 +122,7 @@ int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent)
  *                 Morton bit) or the Karras radix tree over the Morton
  *                 order (0).  Only speed differs, never results
  *   "refill"      persistent ray_fire: idle lanes a wave waits for before
- *                 it claims new work (1..64, default 44)
+ *                 it starts new rays (1..64, default 32)
  *   "fv_refill"   the same for the persistent find_volume (1..64; 0, the
  *                 default: 56 mixed, 40 plain)
  *   "adjoint_sort" adjoint batches of >= 65536 rays with dldv: rays ordered

@@ -1,0 +1,56 @@
+"""Batch sizes at the edges of the resident-grid launches' split: fewer items
+than waves, one item to 64 per wave, exactly the resident lanes, one more
+(the first range from the shared counter), and several ranges per wave with a
+ragged end.  Every size equals the one-item-per-lane kernels bit for bit."""
+import numpy as np
+import pytest
+
+from gpu_util import bits, build_tree, dev, host
+from xdg_amd import geometry as G
+from xdg_amd import philox as P
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+SIZES = [1, 63, 65, 4095, 4097, 100003, 262143, 262144, 262145, 300001, 700001]
+
+
+@pytest.fixture(scope="module")
+def setup():
+    from xdg_amd import capi
+    ctx = capi.Context(0)
+    m = G.nested_spheres(3)
+    vols = list(m.volumes)
+    trees = [build_tree(ctx, m, v) for v in vols]
+    n = max(SIZES)
+    pts = P.box_points(71, P.STREAM_POS, n, [-19] * 3, [19] * 3)
+    lim = min(ctx.tree_info(t)["o_limit"] for t in trees)
+    pts[::997] *= 3.0 * lim / 19.0  # beyond the FP32 boxes' limit
+    dirs = P.iso_dirs(71, P.STREAM_DIR, n)
+    tpr = np.array([trees[i % 5] for i in range(n)], np.int32)
+    tpr[5::1000] = 999  # not a tree
+    yield ctx, m, vols, trees, dev(torch, pts), dev(torch, dirs), dev(torch, tpr)
+    ctx.close()
+
+
+def both_forms(ctx, call):
+    """The result of the per-item and of the resident kernels."""
+    try:
+        ctx.set_traversal(persistent=False)
+        ref = call()
+        ctx.set_traversal(persistent=True)
+        return ref, call()
+    finally:
+        ctx.set_traversal()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", SIZES)
+def test_ray_fire_split(setup, n, prec):
+    ctx, m, vols, trees, pts, dirs, tpr = setup
+    excl = torch.zeros((n, 2), dtype=torch.int32, device="cuda")
+    ref, got = both_forms(ctx, lambda: [host(x) for x in ctx.ray_fire(
+        0, pts[:n], dirs[:n], tree_per_ray=tpr[:n], excl=excl, precision=prec)])
+    assert np.array_equal(bits(got[0]), bits(ref[0]))
+    assert np.array_equal(got[1], ref[1]) and np.array_equal(got[2], ref[2])

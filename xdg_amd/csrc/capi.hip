@@ -338,7 +338,7 @@ LaunchCfg cfg_for(xdg_hip_ctx* c, int depth)
   k.stack = std::max(k.stack, std::max(depth, 1));
   if (k.stack > 64) throw InvalidArg{"tree deeper than the 64-entry traversal stack"};
   // keep the LDS stack within 64 KiB per workgroup
-  while ((size_t)k.stack * k.block * 4 > 65536 && k.block > 64) k.block /= 2;
+  while ((size_t)(k.stack + GUARDED_STACK_EXTRA) * k.block * 4 > 65536 && k.block > 64) k.block /= 2;
   return k;
 }
 

@@ -36,6 +36,15 @@ namespace {
 
 constexpr int MAXK = XDG_HIP_MAX_EXCLUDE;  // exclusion entries per ray (read in place)
 
+// Split of a resident-grid launch (resident_launch).
+struct ResidentCfg {
+  int lanes_first;  // items of a wave's own first range
+  int refill;       // idle lanes of a wave needed before they start new items
+  int min_lanes;    // descend4: lanes that must descend without a leaf for the wave to stay in the node loop
+  int64_t chunk;    // items per range taken from the shared counter
+};
+constexpr int RF_MIN_LANES = 16;
+
 // One ray of ray_fire.  DEFER (mixed only): a ray beyond the FP32-rounding
 // limit is queued for the FP64 pass instead of traced here.
 template <bool MIXED, bool DEFER, bool WIDE, bool SPEC = false>
@@ -98,6 +107,12 @@ __global__ void k_ray_fire_deferred(RayFireArgs a, int cap)
     ray_fire_one<false, false, WIDE>(a, a.fb_list[j], lds + threadIdx.x, cap);
 }
 
+// work counter and deferral count of one launch (either nullable)
+__global__ void k_zero_counters(unsigned long long* next, unsigned int* count)
+{
+  if (next) *next = 0ull;
+  if (count) *count = 0u;
+}
 __global__ void k_zero_u32(unsigned int* p) { *p = 0u; }
 __global__ void k_zero_u64(unsigned long long* p) { *p = 0ull; }
 
@@ -115,132 +130,81 @@ __device__ __forceinline__ void write_hit(const RayFireArgs& a, int64_t i, const
 }
 
 // Persistent ray_fire over the BVH4.  A fixed grid of resident waves works
-// through the batch: a lane whose ray is finished writes its result and
-// takes the next unclaimed ray (one 64-bit atomic per wave per refill), so a
-// wave does not idle behind its slowest lane.  A lane that reaches a leaf
-// while others still descend parks it and keeps descending until every
-// lane holds one (speculative traversal, Aila & Laine 2009).  MIXED queues far-origin rays
-// for the FP64 pass (k_ray_fire_deferred).  Every lane leaves the loop once
-// the counter passes n, so the grid always drains.
+// through the batch; each lane traces one ray at a time as a state machine,
+// and lanes whose ray is done wait until refill_min of their wave are, then
+// write their results and start new rays together (the set-up path is long,
+// and runs for the whole wave).  MIXED queues far-origin rays for the FP64
+// pass (k_ray_fire_deferred).  The loop's control is wave-uniform: a wave
+// leaves once its ranges are dry and every lane is done.
+//
+// What bounds it: VALU issue at about two thirds of the peak and node
+// latency, four waves per SIMD (127 VGPRs).  10 M nested-sphere rays:
+// 2.89 -> 2.19 ms (4 M with FP64 boxes 2.09 -> 1.8), 1 M sphere rays, FP64,
+// 0.456 -> 0.383 ms: ranges per wave instead of one atomic per refill,
+// leaving the node loop when few lanes descend, pushes without branches
+// (wave instructions 110 -> 88 per ray, active lanes 27 -> 37 %).
 template <bool MIXED>
-__device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, int cap, unsigned long long* next_ray,
-                                                 int refill_min)
+__device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, unsigned long long* next_ray,
+                                                 const ResidentCfg& c)
 {
   extern __shared__ int32_t lds[];
-  LdsStack S(lds + threadIdx.x, blockDim.x, cap);
-  const int lane = threadIdx.x & 63;
+  GuardedStack S(lds + threadIdx.x, blockDim.x);
   const int32_t DONE = CHILD_EMPTY;
   int64_t ri = -1;
   bool have = false;  // ri's result is pending
   TreeView T{nullptr, nullptr, nullptr, nullptr};
-  RayD ray;
+  RayD ray{};
   BoxRayF bf{0, 0, 0, 0, 0, 0};
   BoxRayD bd{0, 0, 0, 0, 0, 0};
   HitState h{INFTY, INT32_MAX, ID_NONE, false};
   const int32_t* ex = nullptr;
-  int k = 0;
+  const int k = a.excl ? (a.k < MAXK ? a.k : MAXK) : 0;
   float tf = 0.0f;
   PlaneOfs po{0, 0, 0, 0, 0, 0};
   int32_t node = DONE;
   int32_t leaf = DONE;  // a leaf parked while the wave keeps descending
+  WaveRange w(a.n, c.lanes_first);
   while (true) {
     const bool done = node == DONE && leaf == DONE;
-    if (done && have) {
-      write_hit(a, ri, h);
-      have = false;
-    }
-    // Refill only once enough lanes are idle (or every remaining lane is):
-    // the refill path is long, and running it for one lane at a time costs
-    // the whole wave more than the idle lanes waste.
     const unsigned long long dmask = __ballot(done);
-    const int nact = __popcll(__ballot(1));
-    const bool go = __popcll(dmask) >= (refill_min < nact ? refill_min : nact);
-    const bool need = go && done;
-    const unsigned long long mask = go ? dmask : 0ull;
-    unsigned long long base = 0;
-    if (mask) {
-      const int leader = __ffsll((long long)mask) - 1;
-      unsigned long long b = 0;
-      if (lane == leader) b = atomicAdd(next_ray, (unsigned long long)__popcll(mask));
-      base = __shfl(b, leader);
+    const int nd = __popcll(dmask);
+    if (nd == 64 || (nd >= c.refill && !w.dry)) {
+      if (done && have) {
+        write_hit(a, ri, h);
+        have = false;
+      }
+      if (w.dry) break;  // nd == 64
+      const int64_t slot = w.take(dmask, a.n, c.chunk, c.lanes_first, next_ray);
+      if (done && slot < a.n) {
+        ri = a.order ? (int64_t)a.order[slot] : slot;
+        const int32_t tree = a.tree_per_ray ? a.tree_per_ray[ri] : a.tree;
+        h.t = a.tmax ? a.tmax[ri] : INFTY;
+        h.face = INT32_MAX;
+        h.surf = ID_NONE;
+        h.inside = false;
+        have = true;
+        if (tree >= 1 && tree <= a.ntrees) {
+          const SurfTreeDev& TT = a.table[tree];
+          ray = make_ray(a.org + 3 * ri, a.dir + 3 * ri);
+          if (MIXED && !mixed_safe(TT, ray)) {
+            const unsigned int j = atomicAdd(a.fb_count, 1u);
+            a.fb_list[j] = (int32_t)ri;
+            have = false;
+          } else {
+            T.nodes4_d = TT.nodes4_d;
+            T.nodes4_f = TT.nodes4_f;
+            T.tris = TT.tris;
+            T.normals = TT.normals;
+            ex = a.excl ? a.excl + (int64_t)a.k * ri : nullptr;
+            tf = f32_up(h.t);
+            box_ray<MIXED>(ray, bf, bd, po);
+            S.reset();
+            node = TT.n_prims > 0 ? TT.root4 : DONE;
+          }
+        }
+      }
     }
-    if (need) {
-      const int64_t slot = (int64_t)(base + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull)));
-      if (slot >= a.n) break;
-      ri = a.order ? (int64_t)a.order[slot] : slot;
-      const int32_t tree = a.tree_per_ray ? a.tree_per_ray[ri] : a.tree;
-      if (tree < 1 || tree > a.ntrees) {
-        HitState miss{INFTY, INT32_MAX, ID_NONE, false};
-        write_hit(a, ri, miss);
-        continue;
-      }
-      const SurfTreeDev& TT = a.table[tree];
-      ray = make_ray(a.org + 3 * ri, a.dir + 3 * ri);
-      if (MIXED && !mixed_safe(TT, ray)) {
-        const unsigned int j = atomicAdd(a.fb_count, 1u);
-        a.fb_list[j] = (int32_t)ri;
-        continue;
-      }
-      T.nodes4_d = TT.nodes4_d;
-      T.nodes4_f = TT.nodes4_f;
-      T.tris = TT.tris;
-      T.normals = TT.normals;
-      ex = a.excl ? a.excl + (int64_t)a.k * ri : nullptr;
-      k = a.excl ? (a.k < MAXK ? a.k : MAXK) : 0;
-      h.t = a.tmax ? a.tmax[ri] : INFTY;
-      h.face = INT32_MAX;
-      h.surf = ID_NONE;
-      h.inside = false;
-      tf = f32_up(h.t);
-      if (MIXED) {
-        const float ox = (float)ray.o.x, oy = (float)ray.o.y, oz = (float)ray.o.z;
-        bf.ix = safe_inv_f((float)ray.d.x);
-        bf.iy = safe_inv_f((float)ray.d.y);
-        bf.iz = safe_inv_f((float)ray.d.z);
-        bf.nx = -ox * bf.ix;
-        bf.ny = -oy * bf.iy;
-        bf.nz = -oz * bf.iz;
-      } else {
-        bd.ix = safe_inv_d(ray.d.x);
-        bd.iy = safe_inv_d(ray.d.y);
-        bd.iz = safe_inv_d(ray.d.z);
-        bd.nx = -ray.o.x * bd.ix;
-        bd.ny = -ray.o.y * bd.iy;
-        bd.nz = -ray.o.z * bd.iz;
-      }
-      po = MIXED ? plane_ofs_f(bf) : plane_ofs_d(bd);
-      S.reset();
-      have = true;
-      node = TT.n_prims > 0 ? TT.root4 : DONE;
-      if (node == DONE) continue;
-    }
-    while (node >= 0) {
-      float te[4];
-      int32_t ch[4];
-      node4_test<MIXED>(T, node, bf, bd, po, tf, h.t, te, ch);
-      cswap(te[0], ch[0], te[1], ch[1]);
-      cswap(te[2], ch[2], te[3], ch[3]);
-      cswap(te[0], ch[0], te[2], ch[2]);
-      cswap(te[1], ch[1], te[3], ch[3]);
-      cswap(te[1], ch[1], te[2], ch[2]);
-      if (ch[0] != CHILD_EMPTY) {
-        if (ch[3] != CHILD_EMPTY) S.push(ch[3]);
-        if (ch[2] != CHILD_EMPTY) S.push(ch[2]);
-        if (ch[1] != CHILD_EMPTY) S.push(ch[1]);
-        node = ch[0];
-      } else {
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (node < 0 && node != DONE && leaf == DONE) {
-        leaf = node;
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (__all(leaf != DONE)) break;
-    }
-    if (leaf == DONE && node != DONE) {
-      leaf = node;
-      node = S.empty() ? DONE : S.pop();
-    }
+    descend4<MIXED>(T, S, bf, bd, po, tf, h.t, c.min_lanes, node, leaf);
     if (leaf != DONE) {
       const int32_t first = leaf_first(leaf);
       const int32_t cnt = leaf_count(leaf);
@@ -251,13 +215,13 @@ __device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, int cap, 
   }
 }
 
-__global__ void k_ray_fire_pt_mixed(RayFireArgs a, int cap, unsigned long long* next_ray, int refill_min)
+__global__ void k_ray_fire_pt_mixed(RayFireArgs a, unsigned long long* next_ray, ResidentCfg c)
 {
-  ray_fire_pt_body<true>(a, cap, next_ray, refill_min);
+  ray_fire_pt_body<true>(a, next_ray, c);
 }
-__global__ void k_ray_fire_pt_plain(RayFireArgs a, int cap, unsigned long long* next_ray, int refill_min)
+__global__ void k_ray_fire_pt_plain(RayFireArgs a, unsigned long long* next_ray, ResidentCfg c)
 {
-  ray_fire_pt_body<false>(a, cap, next_ray, refill_min);
+  ray_fire_pt_body<false>(a, next_ray, c);
 }
 
 // Instrumented ray_fire: identical traversal, plus per-ray work counters
@@ -633,6 +597,37 @@ __global__ void k_closest(ClosestArgs a, int cap)
 
 inline dim3 grid1(int64_t n, int blk) { return dim3((unsigned)((n + blk - 1) / blk)); }
 inline size_t lds_bytes(const LaunchCfg& c) { return sizeof(int32_t) * (size_t)c.stack * c.block; }
+inline size_t lds_bytes_guarded(const LaunchCfg& c)
+{
+  return sizeof(int32_t) * (size_t)(c.stack + GUARDED_STACK_EXTRA) * c.block;
+}
+
+// Grid and split of a resident-grid launch over n items, `waves` resident.
+// A batch that gives every wave less than 64 items is spread over all of
+// them: a wave's time is that of its lanes' descents one after another
+// where they diverge, so fewer lanes each end sooner.
+struct ResidentLaunch {
+  unsigned grid;
+  ResidentCfg c;
+  bool counted;  // some items are left for the shared counter
+};
+inline ResidentLaunch resident_launch(int64_t n, int64_t resident_blocks, int block, int refill, int min_lanes)
+{
+  const int64_t wpb = block / 64;
+  const int64_t waves = resident_blocks * wpb;
+  ResidentLaunch L;
+  L.c.lanes_first = (int)std::min<int64_t>(64, std::max<int64_t>(1, (n + waves - 1) / waves));
+  const int64_t need = (n + L.c.lanes_first - 1) / L.c.lanes_first;  // waves
+  L.grid = (unsigned)std::min(resident_blocks, (need + wpb - 1) / wpb);
+  // eight ranges per wave keep the end of the launch balanced; 256 items
+  // amortise the atomic (chunk 64 / 256 / 512: 10 M nested-sphere rays
+  // 2.26 / 2.15 / 2.23 ms, 1 M sphere rays FP64 0.38 / 0.39 / 0.48 ms)
+  L.c.chunk = std::min<int64_t>(256, std::max<int64_t>(64, n / (waves * 8)));
+  L.c.refill = refill;
+  L.c.min_lanes = min_lanes;
+  L.counted = (int64_t)L.grid * wpb * L.c.lanes_first < n;
+  return L;
+}
 
 #define XDG_DISPATCH2(KERNEL, MIXED, WIDE, ...)                                              \
   do {                                                                                       \
@@ -658,17 +653,18 @@ void launch_ray_fire(const RayFireArgs& a, bool mixed, const LaunchCfg& c, hipSt
   const size_t sh = lds_bytes(c);
   const bool persist = (c.persistent & (mixed ? 2 : 1)) != 0;
   if (persist && c.wide && a.next_ray && (!mixed || (a.fb_list && a.fb_count))) {
-    const int64_t need = (a.n + c.block - 1) / c.block;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, a.next_ray);
+    const size_t shg = lds_bytes_guarded(c);
+    const ResidentLaunch L =
+        resident_launch(a.n, mixed ? resident_grid(k_ray_fire_pt_mixed, c.block, shg)
+                                   : resident_grid(k_ray_fire_pt_plain, c.block, shg), c.block, c.refill, RF_MIN_LANES);
+    if (mixed || L.counted)
+      hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(1), 0, s, a.next_ray, mixed ? a.fb_count : nullptr);
     if (mixed) {
-      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, a.fb_count);
-      const int64_t gp = std::min(need, resident_grid(k_ray_fire_pt_mixed, c.block, sh));
-      hipLaunchKernelGGL(k_ray_fire_pt_mixed, dim3((unsigned)gp), b, sh, s, a, c.stack, a.next_ray, c.refill);
-      const unsigned gd = (unsigned)std::min<int64_t>(need, 1024);
+      hipLaunchKernelGGL(k_ray_fire_pt_mixed, dim3(L.grid), b, shg, s, a, a.next_ray, L.c);
+      const unsigned gd = (unsigned)std::min<int64_t>((a.n + c.block - 1) / c.block, 1024);
       hipLaunchKernelGGL((k_ray_fire_deferred<true>), dim3(gd), b, sh, s, a, c.stack);
     } else {
-      const int64_t gp = std::min(need, resident_grid(k_ray_fire_pt_plain, c.block, sh));
-      hipLaunchKernelGGL(k_ray_fire_pt_plain, dim3((unsigned)gp), b, sh, s, a, c.stack, a.next_ray, c.refill);
+      hipLaunchKernelGGL(k_ray_fire_pt_plain, dim3(L.grid), b, shg, s, a, a.next_ray, L.c);
     }
     return;
   }

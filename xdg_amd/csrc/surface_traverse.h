@@ -406,6 +406,146 @@ __device__ __forceinline__ void node4_test(const TT& T, int32_t node, const BoxR
   }
 }
 
+// Traversal stack of the resident-grid kernels, interleaved like LdsStack.
+// Entry 0 of each lane is CHILD_EMPTY for good, so taking from the empty
+// stack gives CHILD_EMPTY; a put writes at the top whatever the value and
+// moves the top only for a child, so a node's pushes need no branches (the
+// branches and execution masks of LdsStack's pushes cost the node loop 3 %:
+// 10 M nested-sphere rays 2.22 -> 2.15 ms).  Callers give it two entries
+// more than the tree's proven stack bound: the guard, and the slot above a
+// full stack that a put of CHILD_EMPTY writes.
+struct GuardedStack {
+  int32_t* top;   // next free
+  int32_t* base;  // top of the empty stack, one entry above the guard
+  int stride;
+  __device__ __forceinline__ GuardedStack(int32_t* b, int s) : top(b + s), base(b + s), stride(s) { *b = CHILD_EMPTY; }
+  __device__ __forceinline__ void reset() { top = base; }
+  __device__ __forceinline__ void put(int32_t v)
+  {
+    *top = v;
+    top += v != CHILD_EMPTY ? stride : 0;
+  }
+  __device__ __forceinline__ int32_t take()
+  {
+    const int32_t v = top[-stride];
+    top -= top != base ? stride : 0;
+    return v;
+  }
+};
+
+// The ray's reciprocal form and plane offsets for one box precision.
+template <bool MIXED>
+__device__ __forceinline__ void box_ray(const RayD& ray, BoxRayF& bf, BoxRayD& bd, PlaneOfs& po)
+{
+  if (MIXED) {
+    const float ox = (float)ray.o.x, oy = (float)ray.o.y, oz = (float)ray.o.z;
+    bf.ix = safe_inv_f((float)ray.d.x);
+    bf.iy = safe_inv_f((float)ray.d.y);
+    bf.iz = safe_inv_f((float)ray.d.z);
+    bf.nx = -ox * bf.ix;
+    bf.ny = -oy * bf.iy;
+    bf.nz = -oz * bf.iz;
+    po = plane_ofs_f(bf);
+  } else {
+    bd.ix = safe_inv_d(ray.d.x);
+    bd.iy = safe_inv_d(ray.d.y);
+    bd.iz = safe_inv_d(ray.d.z);
+    bd.nx = -ray.o.x * bd.ix;
+    bd.ny = -ray.o.y * bd.iy;
+    bd.nz = -ray.o.z * bd.iz;
+    po = plane_ofs_d(bd);
+  }
+}
+
+// Node loop of the resident-grid kernels: lanes descend from `node`; a lane
+// that reaches a leaf parks it in `leaf` and goes on with the next stack
+// entry until it meets a second leaf (speculative traversal, Aila & Laine
+// 2009).  The wave leaves the loop, to test its parked leaves, once fewer
+// than min_lanes lanes descend without a parked leaf: the last few lanes'
+// descents would otherwise run with the rest of the wave idle.  On return
+// a lane holds a leaf, or still an internal node, or is done (both
+// CHILD_EMPTY).
+template <bool MIXED, class STK>
+__device__ __forceinline__ void descend4(const TreeView& T, STK& S, const BoxRayF& bf, const BoxRayD& bd,
+                                         const PlaneOfs& po, float tf, double tm, int min_lanes, int32_t& node,
+                                         int32_t& leaf)
+{
+  while (node >= 0) {
+    float te[4];
+    int32_t ch[4];
+    node4_test<MIXED>(T, node, bf, bd, po, tf, tm, te, ch);
+    cswap(te[0], ch[0], te[1], ch[1]);
+    cswap(te[2], ch[2], te[3], ch[3]);
+    cswap(te[0], ch[0], te[2], ch[2]);
+    cswap(te[1], ch[1], te[3], ch[3]);
+    cswap(te[1], ch[1], te[2], ch[2]);
+    S.put(ch[3]);
+    S.put(ch[2]);
+    S.put(ch[1]);
+    node = ch[0];
+    if (node == CHILD_EMPTY) node = S.take();
+    if (node < 0 && node != CHILD_EMPTY && leaf == CHILD_EMPTY) {
+      leaf = node;
+      node = S.take();
+    }
+    if (__popcll(__ballot(node >= 0 && leaf == CHILD_EMPTY)) < min_lanes) break;
+  }
+  if (node < 0 && node != CHILD_EMPTY && leaf == CHILD_EMPTY) {
+    leaf = node;
+    node = S.take();
+  }
+}
+
+// Work of a resident grid, dealt out per wave.  A wave starts on a range of
+// its own (no atomic), then takes ranges of `chunk` items from one counter
+// and hands their positions to its idle lanes.  One atomic per refill on
+// that counter serialised in its L2 channel (4.8 ns each: 1.1 of the 2.9 ms
+// of 10 M rays), which also made small refills expensive.  beg, end and dry
+// are wave-uniform; take() is called by all lanes of the wave together.
+struct WaveRange {
+  int64_t beg, end;
+  bool dry;  // nothing left to hand out
+  // lanes_first: items of each wave's own first range (<= 64)
+  __device__ __forceinline__ WaveRange(int64_t n, int lanes_first)
+  {
+    const int64_t wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    beg = wave * lanes_first;
+    end = beg + lanes_first < n ? beg + lanes_first : n;
+    dry = beg >= end;
+  }
+  // the position for this lane when it is one of `mask`; n or more: none
+  __device__ __forceinline__ int64_t take(unsigned long long mask, int64_t n, int64_t chunk, int lanes_first,
+                                          unsigned long long* next)
+  {
+    const int lane = threadIdx.x & 63;
+    const int want = __popcll(mask);
+    const int rank = __popcll(mask & ((1ull << lane) - 1ull));
+    const int64_t left = end - beg;
+    const int64_t old = beg + rank;
+    if (want <= left) {
+      beg += want;
+      return old;
+    }
+    // the counter's ranges follow the waves' own first ones
+    const int64_t shared = (int64_t)((gridDim.x * blockDim.x) >> 6) * lanes_first;
+    int64_t nb = n;
+    if (shared < n) {
+      unsigned long long b = 0;
+      if (lane == 0) b = atomicAdd(next, (unsigned long long)chunk);
+      nb = shared + (int64_t)__shfl(b, 0);
+    }
+    if (nb < n) {
+      end = nb + chunk < n ? nb + chunk : n;
+      beg = nb + (want - left) < end ? nb + (want - left) : end;
+      dry = beg == n;
+      return rank < left ? old : nb + (rank - left);
+    }
+    beg = end = n;
+    dry = true;
+    return rank < left ? old : n;
+  }
+};
+
 template <int MODE, bool MIXED, bool STATS, bool SPEC, class STK>
 __device__ __forceinline__ bool traverse4_s(const SurfTreeDev& T, const RayD& ray, int orientation, const int32_t* ex,
                                             int k, STK& S, HitState& h, TraceStats* st = nullptr)

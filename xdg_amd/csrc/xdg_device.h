@@ -494,6 +494,10 @@ __host__ __device__ __forceinline__ int32_t leaf_code(int32_t first, int32_t cou
 __host__ __device__ __forceinline__ int32_t leaf_first(int32_t code) { return (~code) >> 3; }
 __host__ __device__ __forceinline__ int32_t leaf_count(int32_t code) { return ((~code) & 7) + 1; }
 
+// LDS entries per lane a GuardedStack (surface_traverse.h) holds beyond the
+// tree's stack bound.
+constexpr int GUARDED_STACK_EXTRA = 2;
+
 // Per-tree descriptor table entry (device-resident, indexed by tree id).
 struct SurfTreeDev {
   const NodeD* nodes_d;
