@@ -124,7 +124,7 @@ int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent)
  *   "refill"      persistent ray_fire: idle lanes a wave waits for before
  *                 it starts new rays (1..64, default 32)
  *   "fv_refill"   the same for the persistent find_volume (1..64; 0, the
- *                 default: 56 mixed, 40 plain)
+ *                 default: 24)
  *   "adjoint_sort" adjoint batches of >= 65536 rays with dldv: rays ordered
  *                 by hit face and each wave's run on one face summed before
  *                 the vertex atomics (1, default), or nine atomics per ray (0);

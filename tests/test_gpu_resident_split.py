@@ -54,3 +54,11 @@ def test_ray_fire_split(setup, n, prec):
         0, pts[:n], dirs[:n], tree_per_ray=tpr[:n], excl=excl, precision=prec)])
     assert np.array_equal(bits(got[0]), bits(ref[0]))
     assert np.array_equal(got[1], ref[1]) and np.array_equal(got[2], ref[2])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", SIZES)
+def test_find_volume_split(setup, n, prec):
+    ctx, m, vols, trees, pts, dirs, tpr = setup
+    ref, got = both_forms(ctx, lambda: host(ctx.find_volume(trees, vols, m.ipc, pts[:n], dirs[:n], precision=prec)))
+    assert np.array_equal(got, ref)

@@ -44,6 +44,7 @@ struct ResidentCfg {
   int64_t chunk;    // items per range taken from the shared counter
 };
 constexpr int RF_MIN_LANES = 16;
+constexpr int FV_MIN_LANES = 16;
 
 // One ray of ray_fire.  DEFER (mixed only): a ray beyond the FP32-rounding
 // limit is queued for the FP64 pass instead of traced here.
@@ -114,7 +115,6 @@ __global__ void k_zero_counters(unsigned long long* next, unsigned int* count)
   if (count) *count = 0u;
 }
 __global__ void k_zero_u32(unsigned int* p) { *p = 0u; }
-__global__ void k_zero_u64(unsigned long long* p) { *p = 0ull; }
 
 __device__ __forceinline__ void write_hit(const RayFireArgs& a, int64_t i, const HitState& h)
 {
@@ -356,129 +356,88 @@ __global__ void k_find_volume_deferred(FindVolumeArgs a, int cap)
 // point_in_volume traversals volume after volume (a new traversal on the
 // same ray costs only a reset), as a per-lane state machine like the
 // persistent ray_fire: lanes whose traversal has ended record the answer or
-// start the next volume, and claim new points, together once refill_min of
-// the wave are ready, while the other lanes keep descending (with
-// speculative leaf parking).
+// start the next volume, and claim new points, together once c.refill of
+// the wave are ready, while the other lanes keep descending.  Bound by VALU
+// issue like ray_fire.  4 M nested-sphere points, mixed: 3.24 -> 1.92 ms,
+// 0.6 ms of it from ranges per wave and cheap refills, the rest from leaving
+// the node loop below 16 descending lanes (threshold 1 / 8 / 16 / 24: 2.64 /
+// 1.98 / 1.92 / 2.00 ms).
 template <bool MIXED>
-__device__ __forceinline__ void find_volume_pt_body(const FindVolumeArgs& a, int cap, int refill_min)
+__device__ __forceinline__ void find_volume_pt_body(const FindVolumeArgs& a, const ResidentCfg& c)
 {
   extern __shared__ int32_t lds[];
-  LdsStack S(lds + threadIdx.x, blockDim.x, cap);
-  const int lane = threadIdx.x & 63;
+  GuardedStack S(lds + threadIdx.x, blockDim.x);
   const int32_t DONE = CHILD_EMPTY;
   int64_t pi = 0;
   bool hasp = false;   // the lane holds a point whose volume is not known yet
   bool traced = false; // a point_in_volume traversal of volume v is under way or ended
   int v = 0;
   TreeView T{nullptr, nullptr, nullptr, nullptr};
-  RayD ray;
+  RayD ray{};
   BoxRayF bf{0, 0, 0, 0, 0, 0};
   BoxRayD bd{0, 0, 0, 0, 0, 0};
   PlaneOfs po{0, 0, 0, 0, 0, 0};
   HitState h{INFTY, INT32_MAX, ID_NONE, false};
   float tf = INFINITY;
   int32_t node = DONE, leaf = DONE;
+  WaveRange w(a.n, c.lanes_first);
   while (true) {
-    // lanes whose traversal has ended wait until refill_min of the wave (or
-    // all remaining ones) have too; then they act together: record or
+    // lanes whose traversal has ended wait until c.refill of the wave (or
+    // all that still have work) have too; then they act together: record or
     // advance to the next volume, claim new points, start traversals
     const bool done = node == DONE && leaf == DONE;
-    const unsigned long long dmask = __ballot(done);
-    const int nact = __popcll(__ballot(1));
-    const bool go = done && __popcll(dmask) >= (refill_min < nact ? refill_min : nact);
-    if (go && traced) {
-      traced = false;
-      if (h.surf != ID_NONE && h.inside) {
-        a.vol_out[pi] = a.vol_ids[v];
-        hasp = false;
-      } else {
-        ++v;
-      }
-    }
-    const bool need = go && !hasp;
-    const unsigned long long cmask = __ballot(need);
-    if (cmask) {
-      const int leader = __ffsll((long long)cmask) - 1;
-      unsigned long long b = 0;
-      if (lane == leader) b = atomicAdd(a.next, (unsigned long long)__popcll(cmask));
-      b = __shfl(b, leader);
-      if (need) {
-        pi = (int64_t)(b + (unsigned long long)__popcll(cmask & ((1ull << lane) - 1ull)));
-        if (pi >= a.n) break;
-        const double* d = a.dir ? a.dir + 3 * pi : a.dflt;
-        ray = make_ray(a.pts + 3 * pi, d);
-        if (MIXED) {
-          const float ox = (float)ray.o.x, oy = (float)ray.o.y, oz = (float)ray.o.z;
-          bf.ix = safe_inv_f((float)ray.d.x);
-          bf.iy = safe_inv_f((float)ray.d.y);
-          bf.iz = safe_inv_f((float)ray.d.z);
-          bf.nx = -ox * bf.ix;
-          bf.ny = -oy * bf.iy;
-          bf.nz = -oz * bf.iz;
-        } else {
-          bd.ix = safe_inv_d(ray.d.x);
-          bd.iy = safe_inv_d(ray.d.y);
-          bd.iz = safe_inv_d(ray.d.z);
-          bd.nx = -ray.o.x * bd.ix;
-          bd.ny = -ray.o.y * bd.iy;
-          bd.nz = -ray.o.z * bd.iz;
-        }
-        po = MIXED ? plane_ofs_f(bf) : plane_ofs_d(bd);
-        v = 0;
-        hasp = true;
-      }
-    }
-    if (go && hasp) {  // the point's next volume
-      while (v < a.nvol && (a.vol_ids[v] == a.ipc || a.vol_trees[v] < 1 || a.vol_trees[v] > a.ntrees)) ++v;
-      if (v >= a.nvol) {
-        a.vol_out[pi] = a.ipc;
-        hasp = false;
-      } else {
-        const SurfTreeDev& TT = a.table[a.vol_trees[v]];
-        if (MIXED && !mixed_safe(TT, ray)) {  // the whole point goes to the FP64 pass
-          const unsigned int j = atomicAdd(a.fb_count, 1u);
-          a.fb_list[j] = (int32_t)pi;
+    const bool busy = __ballot(!done) != 0;
+    const int ready = __popcll(__ballot(done && (hasp || !w.dry)));
+    if (ready == 0 && !busy) break;
+    if (ready >= c.refill || !busy) {
+      if (done && traced) {
+        traced = false;
+        if (h.surf != ID_NONE && h.inside) {
+          a.vol_out[pi] = a.vol_ids[v];
           hasp = false;
         } else {
-          T.nodes4_d = TT.nodes4_d;
-          T.nodes4_f = TT.nodes4_f;
-          T.tris = TT.tris;
-          T.normals = TT.normals;
-          h = HitState{INFTY, INT32_MAX, ID_NONE, false};
-          tf = INFINITY;
-          S.reset();
-          node = TT.n_prims > 0 ? TT.root4 : DONE;
-          traced = true;
+          ++v;
+        }
+      }
+      const bool need = done && !hasp;
+      const unsigned long long cmask = __ballot(need);
+      if (cmask && !w.dry) {
+        const int64_t pos = w.take(cmask, a.n, c.chunk, c.lanes_first, a.next);
+        if (need && pos < a.n) {
+          pi = pos;
+          const double* d = a.dir ? a.dir + 3 * pi : a.dflt;
+          ray = make_ray(a.pts + 3 * pi, d);
+          box_ray<MIXED>(ray, bf, bd, po);
+          v = 0;
+          hasp = true;
+        }
+      }
+      if (done && hasp) {  // the point's next volume
+        while (v < a.nvol && (a.vol_ids[v] == a.ipc || a.vol_trees[v] < 1 || a.vol_trees[v] > a.ntrees)) ++v;
+        if (v >= a.nvol) {
+          a.vol_out[pi] = a.ipc;
+          hasp = false;
+        } else {
+          const SurfTreeDev& TT = a.table[a.vol_trees[v]];
+          if (MIXED && !mixed_safe(TT, ray)) {  // the whole point goes to the FP64 pass
+            const unsigned int j = atomicAdd(a.fb_count, 1u);
+            a.fb_list[j] = (int32_t)pi;
+            hasp = false;
+          } else {
+            T.nodes4_d = TT.nodes4_d;
+            T.nodes4_f = TT.nodes4_f;
+            T.tris = TT.tris;
+            T.normals = TT.normals;
+            h = HitState{INFTY, INT32_MAX, ID_NONE, false};
+            tf = INFINITY;
+            S.reset();
+            node = TT.n_prims > 0 ? TT.root4 : DONE;
+            traced = true;
+          }
         }
       }
     }
-    while (node >= 0) {
-      float te[4];
-      int32_t ch[4];
-      node4_test<MIXED>(T, node, bf, bd, po, tf, h.t, te, ch);
-      cswap(te[0], ch[0], te[1], ch[1]);
-      cswap(te[2], ch[2], te[3], ch[3]);
-      cswap(te[0], ch[0], te[2], ch[2]);
-      cswap(te[1], ch[1], te[3], ch[3]);
-      cswap(te[1], ch[1], te[2], ch[2]);
-      if (ch[0] != CHILD_EMPTY) {
-        if (ch[3] != CHILD_EMPTY) S.push(ch[3]);
-        if (ch[2] != CHILD_EMPTY) S.push(ch[2]);
-        if (ch[1] != CHILD_EMPTY) S.push(ch[1]);
-        node = ch[0];
-      } else {
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (node < 0 && node != DONE && leaf == DONE) {
-        leaf = node;
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (__all(leaf != DONE)) break;
-    }
-    if (leaf == DONE && node != DONE) {
-      leaf = node;
-      node = S.empty() ? DONE : S.pop();
-    }
+    descend4<MIXED>(T, S, bf, bd, po, tf, h.t, c.min_lanes, node, leaf);
     if (leaf != DONE) {
       const int32_t first = leaf_first(leaf);
       const int32_t cnt = leaf_count(leaf);
@@ -489,14 +448,8 @@ __device__ __forceinline__ void find_volume_pt_body(const FindVolumeArgs& a, int
   }
 }
 
-__global__ void k_find_volume_pt_mixed(FindVolumeArgs a, int cap, int refill_min)
-{
-  find_volume_pt_body<true>(a, cap, refill_min);
-}
-__global__ void k_find_volume_pt_plain(FindVolumeArgs a, int cap, int refill_min)
-{
-  find_volume_pt_body<false>(a, cap, refill_min);
-}
+__global__ void k_find_volume_pt_mixed(FindVolumeArgs a, ResidentCfg c) { find_volume_pt_body<true>(a, c); }
+__global__ void k_find_volume_pt_plain(FindVolumeArgs a, ResidentCfg c) { find_volume_pt_body<false>(a, c); }
 
 template <bool MIXED, bool WIDE>
 __global__ void k_occluded(OccludedArgs a, int cap)
@@ -716,25 +669,25 @@ void launch_find_volume(const FindVolumeArgs& a, bool mixed, const LaunchCfg& c,
   // bit 2 of the persistent mask: the resident grid whose lanes move on to
   // their next volume or point while others still traverse (default), or
   // the per-point kernel that keeps a wave's lanes on the same tree volume
-  // after volume but waits for its longest traversal at each.  The refill
-  // threshold that measured fastest differs by precision (nested spheres,
-  // 10 M points: mixed 7.7 ms at 56, plain 10.4 ms at 40-44).
+  // after volume but waits for its longest traversal at each.  Refill
+  // 8 / 24 / 40 / 56: 1.90 / 1.92 / 2.13 / 3.05 ms mixed (4 M nested-sphere
+  // points), 1.56 / 1.55 / 1.58 / 2.07 ms FP64 (2 M)
   const bool persist = (c.persistent & 4) != 0;
-  const int refill = c.fv_refill ? c.fv_refill : (mixed ? 56 : 40);
+  const int refill = c.fv_refill ? c.fv_refill : 24;
   if (persist && c.wide && a.next && (!mixed || (a.fb_list && a.fb_count))) {
-    const size_t sh = lds_bytes(c);
-    const int64_t need = (a.n + c.block - 1) / c.block;
+    const size_t sh = lds_bytes_guarded(c);
     const dim3 b(c.block);
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, a.next);
+    const ResidentLaunch L =
+        resident_launch(a.n, mixed ? resident_grid(k_find_volume_pt_mixed, c.block, sh)
+                                   : resident_grid(k_find_volume_pt_plain, c.block, sh), c.block, refill, FV_MIN_LANES);
+    if (mixed || L.counted)
+      hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(1), 0, s, a.next, mixed ? a.fb_count : nullptr);
     if (mixed) {
-      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, a.fb_count);
-      const int64_t gp = std::min(need, resident_grid(k_find_volume_pt_mixed, c.block, sh));
-      hipLaunchKernelGGL(k_find_volume_pt_mixed, dim3((unsigned)gp), b, sh, s, a, c.stack, refill);
-      const unsigned gd = (unsigned)std::min<int64_t>(need, 1024);
-      hipLaunchKernelGGL(k_find_volume_deferred, dim3(gd), b, sh, s, a, c.stack);
+      hipLaunchKernelGGL(k_find_volume_pt_mixed, dim3(L.grid), b, sh, s, a, L.c);
+      const unsigned gd = (unsigned)std::min<int64_t>((a.n + c.block - 1) / c.block, 1024);
+      hipLaunchKernelGGL(k_find_volume_deferred, dim3(gd), b, lds_bytes(c), s, a, c.stack);
     } else {
-      const int64_t gp = std::min(need, resident_grid(k_find_volume_pt_plain, c.block, sh));
-      hipLaunchKernelGGL(k_find_volume_pt_plain, dim3((unsigned)gp), b, sh, s, a, c.stack, refill);
+      hipLaunchKernelGGL(k_find_volume_pt_plain, dim3(L.grid), b, sh, s, a, L.c);
     }
     return;
   }
