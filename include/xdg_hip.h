@@ -108,7 +108,8 @@ int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent)
  *   "stack"       minimum LDS stack entries per lane (default 1; raised to
  *                 what each tree needs)
  *   "persistent"  resident-grid kernels: bit 0 plain ray_fire, bit 1 mixed
- *                 ray_fire, bit 2 find_volume (default 7)
+ *                 ray_fire, bit 2 find_volume and point_in_volume
+ *                 (default 7)
  *   "ray_order"   ray_fire batches of >= 65536 rays: 0 caller's order,
  *                 1 sorted by (tree, direction octant, origin Morton code),
  *                 2 as 1 plus one coarse direction bit per axis (0)

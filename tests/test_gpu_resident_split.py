@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-SIZES = [1, 63, 65, 4095, 4097, 100003, 262143, 262144, 262145, 300001, 700001]
+SIZES = [1, 63, 65, 1023, 1025, 4097, 65537, 262143, 262144, 262145, 300001, 700001]
 
 
 @pytest.fixture(scope="module")
@@ -62,3 +62,13 @@ def test_find_volume_split(setup, n, prec):
     ctx, m, vols, trees, pts, dirs, tpr = setup
     ref, got = both_forms(ctx, lambda: host(ctx.find_volume(trees, vols, m.ipc, pts[:n], dirs[:n], precision=prec)))
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", SIZES)
+def test_point_in_volume_split(setup, n, prec):
+    ctx, m, vols, trees, pts, dirs, tpr = setup
+    excl = torch.arange(n, dtype=torch.int32, device="cuda").remainder(2000).reshape(n, 1)
+    for d, ex in ((dirs[:n], excl), (None, None)):
+        ref, got = both_forms(ctx, lambda: host(ctx.point_in_volume(trees[2], pts[:n], d, excl=ex, precision=prec)))
+        assert np.array_equal(got, ref)

@@ -45,6 +45,7 @@ struct ResidentCfg {
 };
 constexpr int RF_MIN_LANES = 16;
 constexpr int FV_MIN_LANES = 16;
+constexpr int PIV_MIN_LANES = 16, PIV_REFILL = 24;
 
 // One ray of ray_fire.  DEFER (mixed only): a ray beyond the FP32-rounding
 // limit is queued for the FP64 pass instead of traced here.
@@ -291,6 +292,76 @@ __global__ void k_piv(PivArgs a, int cap)
   trace<PIV, MIXED, false, WIDE>(T, ray, ORIENT_ANY, ex, k, lds + threadIdx.x, blockDim.x, cap, h);
   a.inside[i] = (h.surf != ID_NONE && h.inside) ? 1 : 0;
 }
+
+// Persistent point_in_volume over the BVH4: the per-lane state machine of
+// the persistent ray_fire with a strided share per wave, so that a launch
+// uses no scratch and may overlap others or be captured.  A point beyond the
+// tree's FP32 limit (mixed) is traced with FP64 boxes at once.  Bound by VALU
+// issue and node latency; the per-point kernel (k_piv) waited for each wave's
+// longest traversal with a quarter of its lanes active.
+// 1 M points in the 163 840-triangle shell: FP64 boxes 650 -> 475 us, mixed
+// 315 us.
+template <bool MIXED>
+__device__ __forceinline__ void piv_pt_body(const PivArgs& a, int cap, const ResidentCfg& c)
+{
+  extern __shared__ int32_t lds[];
+  GuardedStack S(lds + threadIdx.x, blockDim.x);
+  const int32_t DONE = CHILD_EMPTY;
+  int64_t pi = 0;
+  bool have = false;  // pi's answer is pending
+  const SurfTreeDev& TT = a.table[a.tree];
+  const TreeView T{TT.nodes4_d, TT.nodes4_f, TT.tris, TT.normals};
+  const int k = a.excl ? (a.k < MAXK ? a.k : MAXK) : 0;
+  const int32_t* ex = nullptr;
+  RayD ray{};
+  BoxRayF bf{0, 0, 0, 0, 0, 0};
+  BoxRayD bd{0, 0, 0, 0, 0, 0};
+  PlaneOfs po{0, 0, 0, 0, 0, 0};
+  HitState h{INFTY, INT32_MAX, ID_NONE, false};
+  float tf = INFINITY;
+  int32_t node = DONE, leaf = DONE;
+  WaveStride w(a.n, c.lanes_first);
+  while (true) {
+    const bool done = node == DONE && leaf == DONE;
+    const unsigned long long dmask = __ballot(done);
+    const int nd = __popcll(dmask);
+    if (nd == 64 || (nd >= c.refill && !w.dry)) {
+      if (done && have) {
+        a.inside[pi] = (h.surf != ID_NONE && h.inside) ? 1 : 0;
+        have = false;
+      }
+      if (w.dry) break;  // nd == 64
+      const int64_t pos = w.take(dmask, a.n, c.lanes_first);
+      if (done && pos < a.n) {
+        pi = pos;
+        have = true;
+        const double* d = a.dir ? a.dir + 3 * pi : a.dflt;
+        ray = make_ray(a.pts + 3 * pi, d);
+        ex = a.excl ? a.excl + (int64_t)a.k * pi : nullptr;
+        h = HitState{INFTY, INT32_MAX, ID_NONE, false};
+        if (MIXED && !mixed_safe(TT, ray)) {
+          traverse4<PIV, false>(TT, ray, ORIENT_ANY, ex, k, S.base, S.stride, cap, h);
+        } else {
+          tf = INFINITY;
+          box_ray<MIXED>(ray, bf, bd, po);
+          S.reset();
+          node = TT.n_prims > 0 ? TT.root4 : DONE;
+        }
+      }
+    }
+    descend4<MIXED>(T, S, bf, bd, po, tf, h.t, c.min_lanes, node, leaf);
+    if (leaf != DONE) {
+      const int32_t first = leaf_first(leaf);
+      const int32_t cnt = leaf_count(leaf);
+      leaf = DONE;
+      for (int32_t j = 0; j < cnt; ++j) tri_closest_hit<PIV>(T, first + j, ray, ORIENT_ANY, ex, k, h);
+      tf = f32_up(h.t);
+    }
+  }
+}
+
+__global__ void k_piv_pt_mixed(PivArgs a, int cap, ResidentCfg c) { piv_pt_body<true>(a, cap, c); }
+__global__ void k_piv_pt_plain(PivArgs a, int cap, ResidentCfg c) { piv_pt_body<false>(a, cap, c); }
 
 template <bool MIXED, bool WIDE>
 __global__ void k_find_volume(FindVolumeArgs a, int cap, int spec)
@@ -555,10 +626,14 @@ inline size_t lds_bytes_guarded(const LaunchCfg& c)
   return sizeof(int32_t) * (size_t)(c.stack + GUARDED_STACK_EXTRA) * c.block;
 }
 
-// Grid and split of a resident-grid launch over n items, `waves` resident.
-// A batch that gives every wave less than 64 items is spread over all of
-// them: a wave's time is that of its lanes' descents one after another
-// where they diverge, so fewer lanes each end sooner.
+// Grid and split of a resident-grid launch over n items.  A small batch is
+// spread over one wave per SIMD (a quarter of the four resident waves these
+// kernels' registers allow) before a wave gets all its 64 lanes: a wave's
+// time is that of its lanes' descents one after another where they diverge,
+// so fewer lanes each end sooner, until more waves only share a SIMD.
+// Lanes per wave 1 / 4 / 16 / 64, us: 1 000 sphere rays 42 / 41 / 48 / 52,
+// 8 000 point_in_volume 113 / 110 / 113 / 123, 100 000 sphere rays (25 at
+// least) 91 / 89 / 87 / 74.
 struct ResidentLaunch {
   unsigned grid;
   ResidentCfg c;
@@ -569,7 +644,8 @@ inline ResidentLaunch resident_launch(int64_t n, int64_t resident_blocks, int bl
   const int64_t wpb = block / 64;
   const int64_t waves = resident_blocks * wpb;
   ResidentLaunch L;
-  L.c.lanes_first = (int)std::min<int64_t>(64, std::max<int64_t>(1, (n + waves - 1) / waves));
+  const int64_t spread = std::max<int64_t>(1, waves / 4);
+  L.c.lanes_first = (int)std::min<int64_t>(64, (n + spread - 1) / spread);
   const int64_t need = (n + L.c.lanes_first - 1) / L.c.lanes_first;  // waves
   L.grid = (unsigned)std::min(resident_blocks, (need + wpb - 1) / wpb);
   // eight ranges per wave keep the end of the launch balanced; 256 items
@@ -577,7 +653,7 @@ inline ResidentLaunch resident_launch(int64_t n, int64_t resident_blocks, int bl
   // 2.26 / 2.15 / 2.23 ms, 1 M sphere rays FP64 0.38 / 0.39 / 0.48 ms)
   L.c.chunk = std::min<int64_t>(256, std::max<int64_t>(64, n / (waves * 8)));
   L.c.refill = refill;
-  L.c.min_lanes = min_lanes;
+  L.c.min_lanes = std::max(1, min_lanes * L.c.lanes_first / 64);
   L.counted = (int64_t)L.grid * wpb * L.c.lanes_first < n;
   return L;
 }
@@ -660,6 +736,18 @@ void launch_ray_fire_stats(const RayFireArgs& a, bool mixed, const LaunchCfg& c,
 void launch_point_in_volume(const PivArgs& a, bool mixed, const LaunchCfg& c, hipStream_t s)
 {
   if (a.n <= 0) return;
+  if ((c.persistent & 4) && c.wide && a.tree >= 1 && a.tree <= a.ntrees) {
+    const size_t sh = lds_bytes_guarded(c);
+    const int refill = c.fv_refill ? c.fv_refill : PIV_REFILL;
+    const ResidentLaunch L = resident_launch(a.n, mixed ? resident_grid(k_piv_pt_mixed, c.block, sh)
+                                                        : resident_grid(k_piv_pt_plain, c.block, sh), c.block, refill,
+                                             PIV_MIN_LANES);
+    if (mixed)
+      hipLaunchKernelGGL(k_piv_pt_mixed, dim3(L.grid), dim3(c.block), sh, s, a, c.stack, L.c);
+    else
+      hipLaunchKernelGGL(k_piv_pt_plain, dim3(L.grid), dim3(c.block), sh, s, a, c.stack, L.c);
+    return;
+  }
   XDG_DISPATCH2(k_piv, mixed, c.wide, grid1(a.n, c.block), dim3(c.block), lds_bytes(c), s, a, c.stack);
 }
 

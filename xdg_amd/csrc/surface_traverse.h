@@ -546,6 +546,35 @@ struct WaveRange {
   }
 };
 
+// The same without a shared counter, for entry points whose launches may
+// overlap or be captured and so share no scratch: wave w of W takes groups
+// w, w + W, w + 2W, ... of 64 items (or one group of lanes_first items when
+// the batch gives every wave fewer).
+struct WaveStride {
+  int64_t wave, waves, k;  // k: the wave's items handed out so far
+  bool dry;
+  __device__ __forceinline__ int64_t at(int64_t i, int64_t n, int lanes_first) const
+  {
+    if (lanes_first < 64) return i < lanes_first ? wave * lanes_first + i : n;
+    return (((i >> 6) * waves + wave) << 6) + (i & 63);
+  }
+  __device__ __forceinline__ WaveStride(int64_t n, int lanes_first)
+  {
+    wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    waves = (gridDim.x * blockDim.x) >> 6;
+    k = 0;
+    dry = at(0, n, lanes_first) >= n;
+  }
+  __device__ __forceinline__ int64_t take(unsigned long long mask, int64_t n, int lanes_first)
+  {
+    const int lane = threadIdx.x & 63;
+    const int64_t pos = at(k + __popcll(mask & ((1ull << lane) - 1ull)), n, lanes_first);
+    k += __popcll(mask);
+    dry = at(k, n, lanes_first) >= n;
+    return pos;
+  }
+};
+
 template <int MODE, bool MIXED, bool STATS, bool SPEC, class STK>
 __device__ __forceinline__ bool traverse4_s(const SurfTreeDev& T, const RayD& ray, int orientation, const int32_t* ex,
                                             int k, STK& S, HitState& h, TraceStats* st = nullptr)
