@@ -72,3 +72,22 @@ def test_point_in_volume_split(setup, n, prec):
     for d, ex in ((dirs[:n], excl), (None, None)):
         ref, got = both_forms(ctx, lambda: host(ctx.point_in_volume(trees[2], pts[:n], d, excl=ex, precision=prec)))
         assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("n", [1, 3, 65, 4097, 65537, 300001])
+def test_closest_split(setup, n):
+    """closest on a closed shell with points near and far, and at its centre
+    (nearly as far from every triangle: the wave finishes those together)."""
+    import pyoracle as O
+    ctx, m, vols, trees, pts, dirs, tpr = setup
+    p = host(pts)[:n].copy()
+    p[::101] *= 1e-3
+    k = min(n, 4097)
+    for v in (0, 1):
+        d, f = [host(x) for x in ctx.closest(trees[v], dev(torch, p))]
+        rd, rf = O.Tree.from_model(m, vols[v]).closest(p[:k])
+        assert np.array_equal(bits(d[:k]), bits(rd)) and np.array_equal(f[:k], rf)
+        # the other points: the same as in batches of another split
+        for lo in range(k, n, 50000):
+            d2, f2 = [host(x) for x in ctx.closest(trees[v], dev(torch, p[lo:lo + 50000]))]
+            assert np.array_equal(bits(d[lo:lo + 50000]), bits(d2)) and np.array_equal(f[lo:lo + 50000], f2)

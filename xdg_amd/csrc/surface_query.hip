@@ -23,6 +23,7 @@
 // is traced with FP64 boxes (for ray_fire: queued to a second pass so that
 // the mixed kernel carries no FP64 box state).
 #include <algorithm>
+#include <cstddef>
 
 #include "internal.h"
 #include "surface_traverse.h"
@@ -552,70 +553,321 @@ __device__ __forceinline__ double box_d2(const double* b, const D3& p)
   return ex * ex + ey * ey + ez * ez;
 }
 
-__global__ void k_closest(ClosestArgs a, int cap)
+// Is the triangle certainly farther from p than best?  An FP32 distance to
+// its three edges, or to its plane (FP64, stored normal) where p projects
+// inside it, against best^2.  With M the sum of squares of p - v0 and two
+// edges, every FP32 quantity here is off by at most about 10 x 2^-24 M; a
+// projection misjudged as outside lies within 4 x 2^-24 M (squared) of an
+// edge whatever the triangle's shape, and the plane is never farther than
+// the triangle.  The margin is 2^-17 M.  NaN (overflow) answers no.
+// Box distances let about 100 triangles per point pass on a sphere of
+// 20 480 (an inclined triangle's box reaches far beyond it) of which a few
+// need the FP64 closest point, four times this test's work.
+__device__ __forceinline__ bool closest_beyond(const D3& v0, const D3& v1, const D3& v2, const D3& n, const D3& p,
+                                               float best2)
 {
-  extern __shared__ int32_t lds[];
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  double best = INFTY;
-  int32_t bface = INT32_MAX;
-  if (a.tree >= 1 && a.tree <= a.ntrees && a.table[a.tree].n_prims > 0) {
-    const SurfTreeDev& T = a.table[a.tree];
-    const D3 p = d3(a.pts[3 * i], a.pts[3 * i + 1], a.pts[3 * i + 2]);
-    int32_t* stk = lds + threadIdx.x;
-    const int stride = blockDim.x;
-    int sp = 0;
-    int32_t node = T.root;
-    while (true) {
-      if (node >= 0) {
-        const NodeD nd = T.nodes_d[node];
-        double d0 = box_d2(nd.b0, p), d1 = box_d2(nd.b1, p);
-        double lim = best * best;
-        bool h0 = d0 <= lim, h1 = d1 <= lim;
-        int32_t c0 = nd.c0, c1 = nd.c1;
-        if (h0 && h1) {
-          if (d1 < d0) {
-            int32_t tmp = c0;
-            c0 = c1;
-            c1 = tmp;
-          }
-          if (sp < cap) stk[sp++ * stride] = c1;
-          node = c0;
-        } else if (h0) {
-          node = c0;
-        } else if (h1) {
-          node = c1;
-        } else {
-          if (sp == 0) break;
-          node = stk[--sp * stride];
-        }
-        continue;
-      }
-      const int32_t first = leaf_first(node);
-      const int32_t cnt = leaf_count(node);
-      for (int32_t j = 0; j < cnt; ++j) {
-        const TriRec& r = T.tris[first + j];
-        const D3 v0 = d3(r.v[0], r.v[1], r.v[2]);
-        const D3 v1 = d3(r.v[3], r.v[4], r.v[5]);
-        const D3 v2 = d3(r.v[6], r.v[7], r.v[8]);
-        const D3 q = closest_on_triangle(v0, v1, v2, p);
-        const D3 e = sub(q, p);
-        const double dist = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
-        if (dist < best || (dist == best && r.face < bface)) {
-          best = dist;
-          bface = r.face;
-        }
-      }
-      if (sp == 0) break;
-      node = stk[--sp * stride];
+  const D3 d0 = sub(v0, p), d1 = sub(v1, v0), d2 = sub(v2, v0);
+  const double plane = n.x * d0.x + n.y * d0.y + n.z * d0.z;
+  const float wx = (float)d0.x, wy = (float)d0.y, wz = (float)d0.z;
+  const float sx = (float)d1.x, sy = (float)d1.y, sz = (float)d1.z;
+  const float tx = (float)d2.x, ty = (float)d2.y, tz = (float)d2.z;
+  const float pp = wx * wx + wy * wy + wz * wz;
+  const float ss = sx * sx + sy * sy + sz * sz;
+  const float tt = tx * tx + ty * ty + tz * tz;
+  const float st = sx * tx + sy * ty + sz * tz;
+  const float sp = sx * wx + sy * wy + sz * wz;
+  const float tp = tx * wx + ty * wy + tz * wz;
+  const float s = st * tp - tt * sp, t = st * sp - ss * tp;
+  const bool inside = s >= 0.0f && t >= 0.0f && s + t <= ss * tt - st * st;
+  // edges v0v1, v0v2 and v1v2: |w + a e|^2 at the clamped minimum
+  const float a = fminf(fmaxf(-sp * __builtin_amdgcn_rcpf(ss), 0.0f), 1.0f);
+  const float b = fminf(fmaxf(-tp * __builtin_amdgcn_rcpf(tt), 0.0f), 1.0f);
+  const float ee = ss - 2.0f * st + tt, qe = (tp - sp) + (st - ss), qq = pp + 2.0f * sp + ss;
+  const float c = fminf(fmaxf(-qe * __builtin_amdgcn_rcpf(ee), 0.0f), 1.0f);
+  const float e0 = pp + a * (2.0f * sp + a * ss), e1 = pp + b * (2.0f * tp + b * tt), e2 = qq + c * (2.0f * qe + c * ee);
+  const float pl = (float)plane;
+  const float lb = inside ? pl * pl : fminf(fminf(e0, e1), e2);
+  return lb - 0x1p-17f * (pp + ss + tt) > best2;
+}
+
+// The triangles of one leaf against the best distance and face so far (ties:
+// the smaller face).
+__device__ __forceinline__ void closest_tri(const SurfTreeDev& T, int32_t first, int32_t cnt, const D3& p,
+                                            double& best, int32_t& bface)
+{
+  for (int32_t j = 0; j < cnt; ++j) {
+    const auto r = as_global(T.tris + first + j);
+    const auto pn = as_global(T.normals + 3 * (int64_t)(first + j));
+    const D3 v0 = d3(r->v[0], r->v[1], r->v[2]);
+    const D3 v1 = d3(r->v[3], r->v[4], r->v[5]);
+    const D3 v2 = d3(r->v[6], r->v[7], r->v[8]);
+    if (closest_beyond(v0, v1, v2, d3(pn[0], pn[1], pn[2]), p, f32_up(best * best))) continue;
+    const D3 q = closest_on_triangle(v0, v1, v2, p);
+    const D3 e = sub(q, p);
+    const double dist = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
+    const int32_t face = r->face;
+    if (dist < best || (dist == best && face < bface)) {
+      best = dist;
+      bface = face;
     }
   }
-  if (bface == INT32_MAX) {
-    a.dist[i] = INFTY;
-    a.face[i] = ID_NONE;
-  } else {
-    a.dist[i] = best;
-    a.face[i] = bface;
+}
+
+// Distance and face of one point by the binary tree's FP64 boxes: points
+// beyond the FP32 boxes' limit.
+__device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* stk, int stride, int cap, double& best,
+                                    int32_t& bface)
+{
+  int sp = 0;
+  int32_t node = T.root;
+  while (true) {
+    if (node >= 0) {
+      const NodeD nd = T.nodes_d[node];
+      double d0 = box_d2(nd.b0, p), d1 = box_d2(nd.b1, p);
+      double lim = best * best;
+      bool h0 = d0 <= lim, h1 = d1 <= lim;
+      int32_t c0 = nd.c0, c1 = nd.c1;
+      if (h0 && h1) {
+        if (d1 < d0) {
+          int32_t tmp = c0;
+          c0 = c1;
+          c1 = tmp;
+        }
+        if (sp < cap) stk[sp++ * stride] = c1;
+        node = c0;
+      } else if (h0) {
+        node = c0;
+      } else if (h1) {
+        node = c1;
+      } else {
+        if (sp == 0) break;
+        node = stk[--sp * stride];
+      }
+      continue;
+    }
+    closest_tri(T, leaf_first(node), leaf_count(node), p, best, bface);
+    if (sp == 0) break;
+    node = stk[--sp * stride];
+  }
+}
+
+// A point against the BVH4's FP32 boxes.  The boxes were dilated by the
+// tree's bump; pm = p - s and pp = p + s with s just below the bump take that
+// back, so the distance to a box is that to its vertices' bounds.  pm is
+// rounded up and pp down, and the bump loses 2^-40 of the coordinates, more
+// than the rounding of a closest point: only relative roundings are left
+// (one difference, a square, two sums: 5 x 2^-24), which the factor on the
+// limit covers.  A box whose distance exceeds the limit holds no triangle
+// at the best distance or below.
+struct ClosestPointF {
+  float mx, my, mz, px, py, pz;
+};
+__device__ __forceinline__ float closest_limit(double best)
+{
+  return f32_up(best * best) * (1.0f + 0x1p-21f);
+}
+// children within the limit, nearest first (others CHILD_EMPTY)
+__device__ __forceinline__ void node4_dist(const Node4F* nodes, int32_t node, const ClosestPointF& c, float lim,
+                                           float* te, int32_t* ch)
+{
+  const Node4F* nd = nodes + node;
+  const float4 lx = gload_at<float4>(nd, 0u), hx = gload_at<float4>(nd, 16u);
+  const float4 ly = gload_at<float4>(nd, 32u), hy = gload_at<float4>(nd, 48u);
+  const float4 lz = gload_at<float4>(nd, 64u), hz = gload_at<float4>(nd, 80u);
+  const int4 cc = gload_at<int4>(nd, 96u);
+  const float lxa[4] = {lx.x, lx.y, lx.z, lx.w}, hxa[4] = {hx.x, hx.y, hx.z, hx.w};
+  const float lya[4] = {ly.x, ly.y, ly.z, ly.w}, hya[4] = {hy.x, hy.y, hy.z, hy.w};
+  const float lza[4] = {lz.x, lz.y, lz.z, lz.w}, hza[4] = {hz.x, hz.y, hz.z, hz.w};
+  const int32_t cca[4] = {cc.x, cc.y, cc.z, cc.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float ex = fmaxf(fmaxf(lxa[i] - c.mx, c.px - hxa[i]), 0.0f);
+    const float ey = fmaxf(fmaxf(lya[i] - c.my, c.py - hya[i]), 0.0f);
+    const float ez = fmaxf(fmaxf(lza[i] - c.mz, c.pz - hza[i]), 0.0f);
+    const float d = ex * ex + ey * ey + ez * ez;
+    const bool in = d <= lim && cca[i] != CHILD_EMPTY;
+    te[i] = in ? d : INFINITY;
+    ch[i] = in ? cca[i] : CHILD_EMPTY;
+  }
+  cswap(te[0], ch[0], te[1], ch[1]);
+  cswap(te[2], ch[2], te[3], ch[3]);
+  cswap(te[0], ch[0], te[2], ch[2]);
+  cswap(te[1], ch[1], te[3], ch[3]);
+  cswap(te[1], ch[1], te[2], ch[2]);
+}
+
+// LDS of one wave of k_closest: up to 64 points and the queues they share.
+// A queue entry is a child code and a tag: the point's lane, and the upper
+// half of the entry's FP32 box distance (a lower bound).
+constexpr int CLOSEST_NODES = 1536;  // node queue
+constexpr int CLOSEST_LEAVES = 320;  // leaf queue: below 64, plus one step's 4 x 64
+struct ClosestLds {
+  double px[64], py[64], pz[64];
+  unsigned long long best[64];  // bits of the best distance (non-negative: ordered as integers)
+  ClosestPointF c[64];
+  float lim[64];
+  int32_t face[64];
+  int32_t leaf[CLOSEST_LEAVES];
+  uint32_t ltag[CLOSEST_LEAVES];
+  uint32_t ntag[CLOSEST_NODES];
+  int32_t node[CLOSEST_NODES];  // last: also the stacks of closest_fp64
+};
+__device__ __forceinline__ uint32_t closest_tag(int owner, float d)
+{
+  return (__float_as_uint(d) & 0xffff0000u) | (uint32_t)owner;
+}
+__device__ __forceinline__ bool closest_live(uint32_t tag, float lim)
+{
+  return (tag >> 16) <= (__float_as_uint(lim) >> 16);  // non-negative floats order as integers
+}
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Children of one node step into the queues: farther ones first, so that
+// the lanes' nearest children are the next taken.
+__device__ __forceinline__ void closest_push(ClosestLds& L, int owner, const float* te, const int32_t* ch, int& nn,
+                                             int& nl)
+{
+  const unsigned long long below = (1ull << (threadIdx.x & 63)) - 1ull;
+#pragma unroll
+  for (int i = 3; i >= 0; --i) {
+    const bool node = ch[i] >= 0, leaf = ch[i] < 0 && ch[i] != CHILD_EMPTY;
+    const unsigned long long kn = __ballot(node), kl = __ballot(leaf);
+    if (node) {
+      const int k = nn + __popcll(kn & below);
+      L.node[k] = ch[i];
+      L.ntag[k] = closest_tag(owner, te[i]);
+    }
+    if (leaf) {
+      const int k = nl + __popcll(kl & below);
+      L.leaf[k] = ch[i];
+      L.ltag[k] = closest_tag(owner, te[i]);
+    }
+    nn += __popcll(kn);
+    nl += __popcll(kl);
+  }
+}
+
+// closest over the BVH4, one wave per workgroup.  A wave holds up to 64
+// points and works on their descents together: node and leaf entries of all
+// points share two LDS queues, and each step takes up to 64 entries of one
+// queue, one per lane.  A descent per lane left most lanes idle, since
+// points nearly as far from a large part of the surface as from its nearest
+// triangle (the centre of a sphere) visit thousands of nodes where others
+// visit tens; here the wave's lanes share whatever is left.
+//
+// Steps take nodes while fewer than 64 leaves wait, else leaves.  While the
+// node queue has no room for a full step's pushes (3 x 64 net) above
+// `reserve` entries, nodes are taken one at a time: depth first, at most
+// the tree's stack bound more entries, so it cannot overflow.
+// 100 003 points in a ball around a sphere of 20 480 triangles: 7.4 -> 0.35 ms
+// (a descent per lane on these boxes, the last 16 points of a wave finished
+// by all its lanes: 0.73 ms).  Bound by the latency of the steps, two waves
+// per SIMD (19 KB of LDS each).
+__global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int lanes_first)
+{
+  extern __shared__ __align__(16) unsigned char smem[];
+  ClosestLds& L = *(ClosestLds*)smem;
+  const int lane = threadIdx.x;
+  const SurfTreeDev T = a.table[a.tree];
+  double ext = 0.0;
+  for (int k = 0; k < 3; ++k) ext = fmax(ext, fmax(fabs((double)T.box_lo[k]), fabs((double)T.box_hi[k])));
+  const double shrink = T.bump - 0x1p-40 * (ext + T.bump);
+  const double limit = (double)T.o_limit;
+  WaveStride w(a.n, lanes_first);
+  while (!w.dry) {
+    const unsigned long long first = lanes_first < 64 ? (1ull << lanes_first) - 1ull : ~0ull;
+    const int64_t pi = w.take(first, a.n, lanes_first);
+    const bool have = lane < lanes_first && pi < a.n;
+    bool queued = false;
+    if (have) {
+      const D3 p = d3(a.pts[3 * pi], a.pts[3 * pi + 1], a.pts[3 * pi + 2]);
+      double best = INFTY;
+      int32_t bface = INT32_MAX;
+      if (T.n_prims > 0) {
+        if (fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z)) <= limit)
+          queued = true;
+        else
+          closest_fp64(T, p, L.node + lane, 64, reserve, best, bface);
+      }
+      L.px[lane] = p.x;
+      L.py[lane] = p.y;
+      L.pz[lane] = p.z;
+      L.c[lane] = ClosestPointF{f32_up(p.x - shrink),     f32_up(p.y - shrink),     f32_up(p.z - shrink),
+                                f32_down_d(p.x + shrink), f32_down_d(p.y + shrink), f32_down_d(p.z + shrink)};
+      L.best[lane] = (unsigned long long)__double_as_longlong(best);
+      L.face[lane] = bface;
+      L.lim[lane] = INFINITY;
+    }
+    int nn = 0, nl = 0;  // entries in the node and leaf queues
+    {
+      const float te[4] = {0.0f, INFINITY, INFINITY, INFINITY};
+      const int32_t ch[4] = {queued ? T.root4 : CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY};
+      wave_lds_sync();  // every lane's closest_fp64 stack is done with
+      closest_push(L, lane, te, ch, nn, nl);
+    }
+    wave_lds_sync();
+    while (nn + nl > 0) {
+      if (nl < 64 && nn > 0) {
+        const int m = nn + 3 * 64 + reserve <= CLOSEST_NODES ? (nn < 64 ? nn : 64) : 1;
+        float te[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+        int32_t ch[4] = {CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY};
+        int owner = 0;
+        if (lane < m) {
+          const int k = nn - 1 - lane;
+          const uint32_t tag = L.ntag[k];
+          owner = (int)(tag & 63u);
+          const float lim = L.lim[owner];
+          if (closest_live(tag, lim)) node4_dist(T.nodes4_f, L.node[k], L.c[owner], lim, te, ch);
+        }
+        nn -= m;
+        wave_lds_sync();
+        closest_push(L, owner, te, ch, nn, nl);
+      } else {
+        const int m = nl < 64 ? nl : 64;
+        bool cand = false;
+        int owner = 0;
+        double b = INFTY, b0 = INFTY;
+        int32_t f = INT32_MAX;
+        if (lane < m) {
+          const int k = nl - 1 - lane;
+          const uint32_t tag = L.ltag[k];
+          owner = (int)(tag & 63u);
+          if (closest_live(tag, L.lim[owner])) {
+            b = b0 = __longlong_as_double((long long)L.best[owner]);
+            f = L.face[owner];
+            const int32_t f0 = f, code = L.leaf[k];
+            closest_tri(T, leaf_first(code), leaf_count(code), d3(L.px[owner], L.py[owner], L.pz[owner]), b, f);
+            cand = b < b0 || f != f0;
+          }
+        }
+        nl -= m;
+        if (__ballot(cand)) {
+          // several lanes may hold one point's leaves: the least distance
+          // first, then the smallest face at that distance
+          const unsigned long long bits = (unsigned long long)__double_as_longlong(b);
+          if (cand) atomicMin(&L.best[owner], bits);
+          wave_lds_sync();
+          const bool win = cand && L.best[owner] == bits;
+          if (win && b < b0) L.face[owner] = INT32_MAX;
+          wave_lds_sync();
+          if (win) atomicMin(&L.face[owner], f);
+          wave_lds_sync();
+          if (queued) L.lim[lane] = closest_limit(__longlong_as_double((long long)L.best[lane]));
+        }
+      }
+      wave_lds_sync();
+    }
+    if (have) {
+      const int32_t f = L.face[lane];
+      a.dist[pi] = f == INT32_MAX ? INFTY : __longlong_as_double((long long)L.best[lane]);
+      a.face[pi] = f == INT32_MAX ? ID_NONE : f;
+    }
+    wave_lds_sync();
   }
 }
 
@@ -867,7 +1119,13 @@ void launch_occluded(const OccludedArgs& a, bool mixed, const LaunchCfg& c, hipS
 void launch_closest(const ClosestArgs& a, const LaunchCfg& c, hipStream_t s)
 {
   if (a.n <= 0) return;
-  hipLaunchKernelGGL(k_closest, grid1(a.n, c.block), dim3(c.block), lds_bytes(c), s, a, c.stack);
+  const size_t sh = offsetof(ClosestLds, node) + sizeof(int32_t) * (size_t)std::max(CLOSEST_NODES, 64 * c.stack);
+  // spread over every resident wave: its lanes are busy however few points
+  // it holds
+  const int64_t waves = resident_grid(k_closest, 64, sh);
+  const int lanes_first = (int)std::min<int64_t>(64, (a.n + waves - 1) / waves);
+  const unsigned grid = (unsigned)std::min<int64_t>(waves, (a.n + lanes_first - 1) / lanes_first);
+  hipLaunchKernelGGL(k_closest, dim3(grid), dim3(64), sh, s, a, c.stack, lanes_first);
 }
 
 // ---- primitive evaluation (parity checks of the device geometry kernels) --
