@@ -699,6 +699,12 @@ struct HybridStack {
     }
     ++n;
   }
+  // GuardedStack's interface for descend4
+  __device__ __forceinline__ void put(int32_t v)
+  {
+    if (v != CHILD_EMPTY) push(v);
+  }
+  __device__ __forceinline__ int32_t take() { return n == 0 ? CHILD_EMPTY : pop(); }
   __device__ __forceinline__ int32_t pop()
   {
     --n;

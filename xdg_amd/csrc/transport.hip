@@ -29,6 +29,15 @@ using namespace xdgd;
 namespace xdgh {
 namespace {
 
+// Ranges of items and of histories a wave claims at a time, and the node
+// loop's lower bound on descending lanes (descend4).  2^20 histories in the
+// 513-volume lattice, whole launch: event bound 1 / 4 / 8 / 12 / 16 / 24:
+// 9.45 / 8.81 / 8.67 / 8.66 / 8.81 / 8.93 ms; item bound 1 / 8 / 16 / 24:
+// 9.09 / 8.70 / 8.66 / 8.64 ms; histories per claim 64 / 128 / 256: 8.8 /
+// 9.3 / 9.2 ms (histories differ in length, so large ranges end unevenly).
+constexpr int64_t PIV_CHUNK = 256, EVENT_CHUNK = 64;
+constexpr int PIV_MIN_LANES = 16, EVENT_MIN_LANES = 12;
+
 constexpr int HIST = 8;  // exclusion history: last hit faces since the last collision
 enum : uint8_t { TR_ALIVE = 0, TR_ABSORBED, TR_LEAKED, TR_LOST, TR_STUCK, TR_CAPPED, TR_ERROR, TR_VACUUM };
 enum : uint8_t { BC_TRANSMISSION = 0, BC_VACUUM = 1, BC_REFLECTING = 2 };
@@ -442,107 +451,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                                                                                                  TransportRun R)
 {
   extern __shared__ __align__(16) unsigned char smem[];
-  LdsStack S((int32_t*)smem + threadIdx.x, blockDim.x, R.stack_cap);
-  const int lane = threadIdx.x & 63;
+  GuardedStack S((int32_t*)smem + threadIdx.x, blockDim.x);
   const int32_t DONE = CHILD_EMPTY;
   const TransportStage& G = R.stage;
-  const uint64_t total = min((uint64_t)P.slot_cnt[P.nvol], (uint64_t)G.item_cap);
+  const int64_t total = (int64_t)min((uint64_t)P.slot_cnt[P.nvol], (uint64_t)G.item_cap);
   bool traced = false;
   int2 it = make_int2(0, 0);
   TreeView T{nullptr, nullptr, nullptr, nullptr};
-  RayD ray;
+  RayD ray{};
   BoxRayF bf{0, 0, 0, 0, 0, 0};
   BoxRayD bd{0, 0, 0, 0, 0, 0};
   PlaneOfs po{0, 0, 0, 0, 0, 0};
   HitState h{INFTY, INT32_MAX, ID_NONE, false};
   float tf = 0.0f;
   int32_t node = DONE, leaf = DONE;
+  WaveRange w(total, 64);
   while (true) {
     const bool done = node == DONE && leaf == DONE;
     const unsigned long long dmask = __ballot(done);
-    const int nact = __popcll(__ballot(1));
-    const bool go = done && __popcll(dmask) >= (R.refill < nact ? R.refill : nact);
-    if (go && traced) {
-      traced = false;
-      if (h.surf != ID_NONE && h.inside) atomicMin(G.found + it.x, it.y);
-    }
-    const unsigned long long cmask = __ballot(go);
-    if (cmask) {
-      const int leader = __ffsll((long long)cmask) - 1;
-      unsigned long long b = 0;
-      if (lane == leader) b = atomicAdd(G.claim, (unsigned long long)__popcll(cmask));
-      b = __shfl(b, leader);
-      if (go) {
-        const uint64_t k = b + (unsigned long long)__popcll(cmask & ((1ull << lane) - 1ull));
-        if (k >= total) break;
+    const int nd = __popcll(dmask);
+    if (nd == 64 || (nd >= R.refill && !w.dry)) {
+      if (done && traced) {
+        traced = false;
+        if (h.surf != ID_NONE && h.inside) atomicMin(G.found + it.x, it.y);
+      }
+      if (w.dry) break;  // nd == 64
+      const int64_t k = w.take(dmask, total, PIV_CHUNK, 64, G.claim);
+      if (done && k < total) {
         it = G.items[k];
         // an item whose history holds a lower containing slot cannot lower
         // the minimum: skipped (no result depends on the skip)
-        if (G.over[it.x] || __hip_atomic_load(G.found + it.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < it.y)
-          continue;
-        const SurfTreeDev& TT = P.table[P.vol_tree[it.y]];
-        D3 r, u;
-        load_start(G, it.x, r, u);
-        ray = make_ray_d3(r, u);
-        h = HitState{INFTY, INT32_MAX, ID_NONE, false};
-        T.nodes4_d = TT.nodes4_d;
-        T.nodes4_f = TT.nodes4_f;
-        T.tris = TT.tris;
-        T.normals = TT.normals;
-        traced = true;
-        S.reset();
-        if (MIXED && !mixed_safe(TT, ray)) {
-          trace_s<PIV, false>(TT, ray, ORIENT_ANY, nullptr, 0, S, h);
-          continue;
+        if (!G.over[it.x] && __hip_atomic_load(G.found + it.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= it.y) {
+          const SurfTreeDev& TT = P.table[P.vol_tree[it.y]];
+          D3 r, u;
+          load_start(G, it.x, r, u);
+          ray = make_ray_d3(r, u);
+          h = HitState{INFTY, INT32_MAX, ID_NONE, false};
+          T.nodes4_d = TT.nodes4_d;
+          T.nodes4_f = TT.nodes4_f;
+          T.tris = TT.tris;
+          T.normals = TT.normals;
+          traced = true;
+          if (MIXED && !mixed_safe(TT, ray)) {
+            traverse4<PIV, false>(TT, ray, ORIENT_ANY, nullptr, 0, S.base, S.stride, R.stack_cap, h);
+          } else {
+            box_ray<MIXED>(ray, bf, bd, po);
+            tf = f32_up(h.t);
+            S.reset();
+            node = TT.n_prims > 0 ? TT.root4 : DONE;
+          }
         }
-        if (MIXED) {
-          const float ox = (float)ray.o.x, oy = (float)ray.o.y, oz = (float)ray.o.z;
-          bf.ix = safe_inv_f((float)ray.d.x);
-          bf.iy = safe_inv_f((float)ray.d.y);
-          bf.iz = safe_inv_f((float)ray.d.z);
-          bf.nx = -ox * bf.ix;
-          bf.ny = -oy * bf.iy;
-          bf.nz = -oz * bf.iz;
-        } else {
-          bd.ix = safe_inv_d(ray.d.x);
-          bd.iy = safe_inv_d(ray.d.y);
-          bd.iz = safe_inv_d(ray.d.z);
-          bd.nx = -ray.o.x * bd.ix;
-          bd.ny = -ray.o.y * bd.iy;
-          bd.nz = -ray.o.z * bd.iz;
-        }
-        po = MIXED ? plane_ofs_f(bf) : plane_ofs_d(bd);
-        tf = f32_up(h.t);
-        node = TT.n_prims > 0 ? TT.root4 : DONE;
       }
     }
-    while (node >= 0) {
-      float te[4];
-      int32_t ch[4];
-      node4_test<MIXED>(T, node, bf, bd, po, tf, h.t, te, ch);
-      cswap(te[0], ch[0], te[1], ch[1]);
-      cswap(te[2], ch[2], te[3], ch[3]);
-      cswap(te[0], ch[0], te[2], ch[2]);
-      cswap(te[1], ch[1], te[3], ch[3]);
-      cswap(te[1], ch[1], te[2], ch[2]);
-      if (ch[0] != CHILD_EMPTY) {
-        if (ch[3] != CHILD_EMPTY) S.push(ch[3]);
-        if (ch[2] != CHILD_EMPTY) S.push(ch[2]);
-        if (ch[1] != CHILD_EMPTY) S.push(ch[1]);
-        node = ch[0];
-      } else {
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (node < 0 && node != DONE && leaf == DONE) {
-        leaf = node;
-        node = S.empty() ? DONE : S.pop();
-      }
-      if (__all(leaf != DONE)) break;
-    }
-    if (leaf == DONE && node != DONE) {
-      leaf = node;
-      node = S.empty() ? DONE : S.pop();
-    }
+    descend4<MIXED>(T, S, bf, bd, po, tf, h.t, PIV_MIN_LANES, node, leaf);
     if (leaf != DONE) {
       const int32_t first = leaf_first(leaf);
       const int32_t cnt = leaf_count(leaf);
@@ -885,122 +846,77 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 {
   extern __shared__ __align__(16) unsigned char smem[];
   EventLds E = event_lds(smem, P, R);
-  const int lane = threadIdx.x & 63;
   const int32_t DONE = CHILD_EMPTY;
-  const uint64_t n = R.rounds > 0 ? (uint64_t)*R.stage.live : (uint64_t)R.n;
+  const int64_t n = R.rounds > 0 ? (int64_t)*R.stage.live : R.n;
   bool have = false;    // the lane holds a live history
   bool traced = false;  // its current event's ray is traced (or being traced)
   int64_t hix = 0;
   Hist H;
   H.st = TR_ALIVE;
   TreeView T{nullptr, nullptr, nullptr, nullptr};
-  RayD ray;
+  RayD ray{};
   BoxRayF bf{0, 0, 0, 0, 0, 0};
   BoxRayD bd{0, 0, 0, 0, 0, 0};
   PlaneOfs po{0, 0, 0, 0, 0, 0};
   HitState h{INFTY, INT32_MAX, ID_NONE, false};
   float tf = 0.0f;
   int32_t node = DONE, leaf = DONE, slot = -1;
+  WaveRange w(n, 64);
   while (true) {
     const bool done = node == DONE && leaf == DONE;
-    const unsigned long long dmask = __ballot(done);
-    const int nact = __popcll(__ballot(1));
-    const bool go = done && __popcll(dmask) >= (R.refill < nact ? R.refill : nact);
-    if (go && traced) {
-      traced = false;
-      event_finish(P, R, E.ltally, E.hist, H, h, T.normals, slot);
-      if (H.st != TR_ALIVE) {
-        record_end(R, hix, H);
-        have = false;
+    const bool busy = __ballot(!done) != 0;
+    const int ready = __popcll(__ballot(done && (have || !w.dry)));
+    if (ready == 0 && !busy) break;
+    if (ready >= R.refill || !busy) {
+      if (done && traced) {
+        traced = false;
+        event_finish(P, R, E.ltally, E.hist, H, h, T.normals, slot);
+        if (H.st != TR_ALIVE) {
+          record_end(R, hix, H);
+          have = false;
+        }
+      }
+      // lanes without a history claim the next ones of the list
+      const bool need = done && !have;
+      const unsigned long long cmask = __ballot(need);
+      if (cmask && !w.dry) {
+        const int64_t pos = w.take(cmask, n, EVENT_CHUNK, 64, R.next);
+        if (need && pos < n) {
+          hix = (int64_t)R.stage.idx[pos];
+          load_hist(R, hix, H, E.hist);
+          have = H.st == TR_ALIVE;  // one that ended at its start has its record already
+        }
+      }
+      // lanes with a live history and no ray start the next event's ray
+      if (done && have) {
+        int32_t t;
+        slot = event_slot(P, H, t);
+        if (slot < 0) {
+          H.st = TR_ERROR;
+          record_end(R, hix, H);
+          have = false;
+        } else {
+          const SurfTreeDev& TT = P.table[t];
+          ray = make_ray_d3(H.r, H.u);
+          h = HitState{INFTY, INT32_MAX, ID_NONE, false};
+          T.nodes4_d = TT.nodes4_d;
+          T.nodes4_f = TT.nodes4_f;
+          T.tris = TT.tris;
+          T.normals = TT.normals;
+          traced = true;
+          E.S.reset();
+          if (MIXED && !mixed_safe(TT, ray)) {
+            // an origin beyond the tree's FP32 limit: FP64 boxes, traced at once
+            trace_s<RAYFIRE, false>(TT, ray, ORIENT_EXITING, E.hist, H.hn, E.S, h);
+          } else {
+            box_ray<MIXED>(ray, bf, bd, po);
+            tf = f32_up(h.t);
+            node = TT.n_prims > 0 ? TT.root4 : DONE;
+          }
+        }
       }
     }
-    // lanes without a history claim the next ones of the list
-    const bool need = go && !have;
-    const unsigned long long cmask = __ballot(need);
-    if (cmask) {
-      const int leader = __ffsll((long long)cmask) - 1;
-      unsigned long long b = 0;
-      if (lane == leader) b = atomicAdd(R.next, (unsigned long long)__popcll(cmask));
-      b = __shfl(b, leader);
-      if (need) {
-        const uint64_t pos = b + (unsigned long long)__popcll(cmask & ((1ull << lane) - 1ull));
-        if (pos >= n) break;
-        hix = (int64_t)R.stage.idx[pos];
-        load_hist(R, hix, H, E.hist);
-        have = H.st == TR_ALIVE;  // one that ended at its start has its record already
-      }
-    }
-    // lanes with a live history and no ray start the next event's ray
-    if (go && have) {
-      int32_t t;
-      slot = event_slot(P, H, t);
-      if (slot < 0) {
-        H.st = TR_ERROR;
-        record_end(R, hix, H);
-        have = false;
-        continue;
-      }
-      const SurfTreeDev& TT = P.table[t];
-      ray = make_ray_d3(H.r, H.u);
-      h = HitState{INFTY, INT32_MAX, ID_NONE, false};
-      T.nodes4_d = TT.nodes4_d;
-      T.nodes4_f = TT.nodes4_f;
-      T.tris = TT.tris;
-      T.normals = TT.normals;
-      traced = true;
-      E.S.reset();
-      if (MIXED && !mixed_safe(TT, ray)) {
-        // an origin beyond the tree's FP32 limit: FP64 boxes, traced at once
-        trace_s<RAYFIRE, false>(TT, ray, ORIENT_EXITING, E.hist, H.hn, E.S, h);
-        continue;
-      }
-      if (MIXED) {
-        const float ox = (float)ray.o.x, oy = (float)ray.o.y, oz = (float)ray.o.z;
-        bf.ix = safe_inv_f((float)ray.d.x);
-        bf.iy = safe_inv_f((float)ray.d.y);
-        bf.iz = safe_inv_f((float)ray.d.z);
-        bf.nx = -ox * bf.ix;
-        bf.ny = -oy * bf.iy;
-        bf.nz = -oz * bf.iz;
-      } else {
-        bd.ix = safe_inv_d(ray.d.x);
-        bd.iy = safe_inv_d(ray.d.y);
-        bd.iz = safe_inv_d(ray.d.z);
-        bd.nx = -ray.o.x * bd.ix;
-        bd.ny = -ray.o.y * bd.iy;
-        bd.nz = -ray.o.z * bd.iz;
-      }
-      po = MIXED ? plane_ofs_f(bf) : plane_ofs_d(bd);
-      tf = f32_up(h.t);
-      node = TT.n_prims > 0 ? TT.root4 : DONE;
-    }
-    while (node >= 0) {
-      float te[4];
-      int32_t ch[4];
-      node4_test<MIXED>(T, node, bf, bd, po, tf, h.t, te, ch);
-      cswap(te[0], ch[0], te[1], ch[1]);
-      cswap(te[2], ch[2], te[3], ch[3]);
-      cswap(te[0], ch[0], te[2], ch[2]);
-      cswap(te[1], ch[1], te[3], ch[3]);
-      cswap(te[1], ch[1], te[2], ch[2]);
-      if (ch[0] != CHILD_EMPTY) {
-        if (ch[3] != CHILD_EMPTY) E.S.push(ch[3]);
-        if (ch[2] != CHILD_EMPTY) E.S.push(ch[2]);
-        if (ch[1] != CHILD_EMPTY) E.S.push(ch[1]);
-        node = ch[0];
-      } else {
-        node = E.S.empty() ? DONE : E.S.pop();
-      }
-      if (node < 0 && node != DONE && leaf == DONE) {
-        leaf = node;
-        node = E.S.empty() ? DONE : E.S.pop();
-      }
-      if (__all(leaf != DONE)) break;
-    }
-    if (leaf == DONE && node != DONE) {
-      leaf = node;
-      node = E.S.empty() ? DONE : E.S.pop();
-    }
+    descend4<MIXED>(T, E.S, bf, bd, po, tf, h.t, EVENT_MIN_LANES, node, leaf);
     if (leaf != DONE) {
       const int32_t first = leaf_first(leaf);
       const int32_t cnt = leaf_count(leaf);
@@ -1128,7 +1044,10 @@ TransportLaunch transport_shape(bool mixed, int block, int lds_stack, int nvol)
   return L;
 }
 
-size_t transport_start_lds(int block, int stack_cap) { return (size_t)block * 4 * (size_t)stack_cap; }
+size_t transport_start_lds(int block, int stack_cap)
+{
+  return (size_t)block * 4 * (size_t)(stack_cap + GUARDED_STACK_EXTRA);
+}
 
 int transport_start_block(int stack_cap)
 {
