@@ -91,3 +91,21 @@ def test_closest_split(setup, n):
         for lo in range(k, n, 50000):
             d2, f2 = [host(x) for x in ctx.closest(trees[v], dev(torch, p[lo:lo + 50000]))]
             assert np.array_equal(bits(d[lo:lo + 50000]), bits(d2)) and np.array_equal(f[lo:lo + 50000], f2)
+
+
+@pytest.mark.parametrize("n", [1, 63, 1025, 65537, 300001])
+def test_find_element_split(setup, n):
+    """Points inside, on lattice planes and outside the mesh; every batch
+    size equals the oracle on its first points and smaller batches beyond."""
+    import pyoracle as O
+    ctx = setup[0]
+    mesh = G.kuhn_cube(7, 0.2, seed=4)
+    et = ctx.build_element_tree(mesh.verts, mesh.tets, mesh.adj, mesh.face_order)
+    p = P.box_points(73, P.STREAM_POS, n, [-0.1] * 3, [1.1] * 3)
+    p[::7] = np.round(p[::7] * 7) / 7
+    k = min(n, 20000)
+    got = host(ctx.find_element(et, dev(torch, p)))
+    om = O.TetMesh(mesh, with_ipc=False)
+    assert np.array_equal(got[:k], om.find_element(p[:k]))
+    for lo in range(k, n, 50000):
+        assert np.array_equal(got[lo:lo + 50000], host(ctx.find_element(et, dev(torch, p[lo:lo + 50000]))))

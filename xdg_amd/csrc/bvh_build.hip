@@ -37,6 +37,16 @@ void* dev_alloc(size_t bytes, std::vector<DevBuf>& owned)
   return p;
 }
 
+void dev_free_one(std::vector<DevBuf>& owned, void* p)
+{
+  for (auto it = owned.begin(); p && it != owned.end(); ++it)
+    if (it->p == p) {
+      (void)hipFree(p);
+      owned.erase(it);
+      return;
+    }
+}
+
 void dev_free_all(std::vector<DevBuf>& owned)
 {
   for (auto& b : owned)
@@ -1167,7 +1177,7 @@ __global__ void k_c4_emit(const NodeD* __restrict__ nd, const NodeF* __restrict_
       if (src4) src4[4 * (int64_t)it.slot + j] = -1;
     }
   }
-  o4d[it.slot] = d4;
+  if (o4d) o4d[it.slot] = d4;
   o4f[it.slot] = f4;
 }
 
@@ -1207,13 +1217,13 @@ __global__ void k_copy_bytes16(const uint4* __restrict__ src, uint4* dst, int64_
 }  // namespace
 
 void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<DevBuf>& owned, Bvh4Out& out,
-                   bool keep_sources)
+                   bool keep_sources, bool fp64_nodes)
 {
   if (bin.root < 0 || bin.n_nodes == 0) {  // a single leaf: no nodes
     out.root = bin.root;
     out.stack = 0;
     out.n_nodes = 0;
-    out.nodes_d = (Node4D*)dev_alloc(sizeof(Node4D), owned);
+    if (fp64_nodes) out.nodes_d = (Node4D*)dev_alloc(sizeof(Node4D), owned);
     out.nodes_f = (Node4F*)dev_alloc(sizeof(Node4F), owned);
     return;
   }
@@ -1221,7 +1231,7 @@ void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<Dev
   try {
     // a 4-wide node absorbs at least one binary node: n_nodes bounds the count
     const int64_t cap = bin.n_nodes;
-    auto* t4d = (Node4D*)dev_alloc(sizeof(Node4D) * (size_t)cap, tmp);
+    Node4D* t4d = fp64_nodes ? (Node4D*)dev_alloc(sizeof(Node4D) * (size_t)cap, tmp) : nullptr;
     auto* t4f = (Node4F*)dev_alloc(sizeof(Node4F) * (size_t)cap, tmp);
     int32_t* tsrc = keep_sources ? (int32_t*)dev_alloc(sizeof(int32_t) * 4 * (size_t)cap, tmp) : nullptr;
     auto* lv0 = (C4Item*)dev_alloc(sizeof(C4Item) * (size_t)cap, tmp);
@@ -1259,9 +1269,10 @@ void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<Dev
     if (h[1] & 4u) throw HipError{"bvh4: a primitive is not covered exactly once"};
     // right-sized final arrays, copied on the device
     out.n_nodes = slots;
-    out.nodes_d = (Node4D*)dev_alloc(sizeof(Node4D) * (size_t)slots, owned);
+    if (fp64_nodes) out.nodes_d = (Node4D*)dev_alloc(sizeof(Node4D) * (size_t)slots, owned);
     out.nodes_f = (Node4F*)dev_alloc(sizeof(Node4F) * (size_t)slots, owned);
-    XDG_HIP_CHECK(hipMemcpyAsync(out.nodes_d, t4d, sizeof(Node4D) * (size_t)slots, hipMemcpyDeviceToDevice, s));
+    if (fp64_nodes)
+      XDG_HIP_CHECK(hipMemcpyAsync(out.nodes_d, t4d, sizeof(Node4D) * (size_t)slots, hipMemcpyDeviceToDevice, s));
     XDG_HIP_CHECK(hipMemcpyAsync(out.nodes_f, t4f, sizeof(Node4F) * (size_t)slots, hipMemcpyDeviceToDevice, s));
     if (keep_sources) {
       out.src = (int32_t*)dev_alloc(sizeof(int32_t) * 4 * (size_t)slots, owned);

@@ -70,7 +70,8 @@ struct GraphHandle {
 struct ElemTreeHost {
   ElemTreeDev dev{};
   std::vector<DevBuf> bufs;
-  int64_t n_nodes = 0;
+  int64_t n_nodes = 0;  // of the binary tree (depth and root too)
+  int32_t depth = 0, root = 0;
   int64_t bytes = 0;
   int64_t n_bfaces = 0;
 };
@@ -138,7 +139,6 @@ struct xdg_hip_ctx {
   int refit = 0;  // surface trees built next keep what a refit needs
   int max_surf_depth = 1;
   int max_surf_stack4 = 1;
-  int max_elem_depth = 1;
 };
 
 namespace {
@@ -839,13 +839,18 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
       lbvh_build(d_box, n_tets, c->leaf_max, s, t.bufs, lb, false, c->build_sah != 0);
       XDG_HIP_CHECK(hipGetLastError());
       XDG_HIP_CHECK(hipStreamSynchronize(s));
-      t.dev.nodes_d = lb.nodes_d;
-      t.dev.nodes_f = lb.nodes_f;
+      Bvh4Out b4;
+      bvh4_collapse(lb, n_tets, s, t.bufs, b4, false, false);
+      // queries read the FP32 BVH4 alone
+      for (void* p : {(void*)lb.nodes_d, (void*)lb.nodes_f}) dev_free_one(t.bufs, p);
+      t.dev.nodes4_f = b4.nodes_f;
       t.dev.order = lb.order;
       t.dev.elems = d_elems;
-      t.dev.root = lb.root;
+      t.dev.root4 = b4.root;
+      t.dev.stack4 = b4.stack;
+      t.depth = lb.depth;
+      t.root = lb.root;
       t.dev.n_prims = (int32_t)n_tets;
-      t.dev.depth = lb.depth;
       for (int f = 0; f < 12; ++f) t.dev.face_order[f] = face_order ? face_order[f] : 0;
       t.dev.ipc_tree = -1;
       for (int k = 0; k < 3; ++k) {
@@ -868,8 +873,7 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
     }
     dev_free_all(tmp);
     c->elem.push_back(std::move(t));
-    c->max_elem_depth = std::max(c->max_elem_depth, c->elem.back().dev.depth);
-    try {
+      try {
       sync_tables(c);
     } catch (...) {
       dev_free_all(c->elem.back().bufs);
@@ -912,8 +916,8 @@ int xdg_hip_get_tree_info(xdg_hip_ctx* c, int32_t tree, int element, xdg_hip_tre
       const ElemTreeHost& t = elem_tree(c, tree);
       info->n_prims = t.dev.n_prims;
       info->n_nodes = t.n_nodes;
-      info->depth = t.dev.depth;
-      info->root = t.dev.root;
+      info->depth = t.depth;
+      info->root = t.root;
       info->bytes = t.bytes;
       info->bump = 0.0;
       info->o_limit = 0.0;
@@ -1313,7 +1317,7 @@ int xdg_hip_find_element(xdg_hip_ctx* c, int32_t element_tree, int64_t n, const 
     if (n == 0) return XDG_HIP_OK;
     require(pts && elem_out, "null array");
     FindElementArgs a{c->d_elem, (int32_t)c->elem.size(), element_tree, n, pts, elem_out};
-    launch_find_element(a, cfg_for(c, t.dev.depth), pick(c, stream));
+    launch_find_element(a, cfg_for(c, t.dev.stack4), pick(c, stream));
     XDG_HIP_CHECK(hipGetLastError());
     return XDG_HIP_OK;
   });
@@ -1341,7 +1345,7 @@ int xdg_hip_tally_segments(xdg_hip_ctx* c, int32_t element_tree, int64_t n, cons
   return guarded(c, [&]() {
     require(n >= 0, "negative n");
     const ElemTreeHost& t = elem_tree(c, element_tree);
-    int depth = t.dev.depth;
+    int depth = t.dev.stack4;
     if (t.dev.ipc_tree >= 1) depth = std::max(depth, surf_tree(c, t.dev.ipc_tree).dev.depth);
     if (n == 0) return XDG_HIP_OK;
     require(p0 && p1 && count_out && hash_out, "null array");
@@ -1384,7 +1388,7 @@ int xdg_hip_tally_segments_volume(xdg_hip_ctx* c, int32_t element_tree, int32_t 
   return guarded(c, [&]() {
     require(n >= 0, "negative n");
     const ElemTreeHost& t = elem_tree(c, element_tree);
-    int depth = t.dev.depth;
+    int depth = t.dev.stack4;
     depth = std::max(depth, surf_tree(c, surface_tree).dev.depth);
     if (n == 0) return XDG_HIP_OK;
     require(p0 && p1 && count_out && hash_out, "null array");
@@ -1426,7 +1430,7 @@ int xdg_hip_mesh_walk(xdg_hip_ctx* c, int32_t element_tree, uint64_t first, int6
     require(std::isfinite(mfp) && mfp > 0.0, "mfp must be finite and > 0");
     require(max_events >= 1, "max_events must be >= 1");
     const ElemTreeHost& t = elem_tree(c, element_tree);
-    int depth = t.dev.depth;
+    int depth = t.dev.stack4;
     if (t.dev.ipc_tree >= 1) depth = std::max(depth, surf_tree(c, t.dev.ipc_tree).dev.depth);
     if (n == 0) return XDG_HIP_OK;
     MeshWalkArgs a{};

@@ -37,13 +37,6 @@ namespace {
 
 constexpr int MAXK = XDG_HIP_MAX_EXCLUDE;  // exclusion entries per ray (read in place)
 
-// Split of a resident-grid launch (resident_launch).
-struct ResidentCfg {
-  int lanes_first;  // items of a wave's own first range
-  int refill;       // idle lanes of a wave needed before they start new items
-  int min_lanes;    // descend4: lanes that must descend without a leaf for the wave to stay in the node loop
-  int64_t chunk;    // items per range taken from the shared counter
-};
 constexpr int RF_MIN_LANES = 16;
 constexpr int FV_MIN_LANES = 16;
 constexpr int PIV_MIN_LANES = 16, PIV_REFILL = 24;
@@ -876,38 +869,6 @@ inline size_t lds_bytes(const LaunchCfg& c) { return sizeof(int32_t) * (size_t)c
 inline size_t lds_bytes_guarded(const LaunchCfg& c)
 {
   return sizeof(int32_t) * (size_t)(c.stack + GUARDED_STACK_EXTRA) * c.block;
-}
-
-// Grid and split of a resident-grid launch over n items.  A small batch is
-// spread over one wave per SIMD (a quarter of the four resident waves these
-// kernels' registers allow) before a wave gets all its 64 lanes: a wave's
-// time is that of its lanes' descents one after another where they diverge,
-// so fewer lanes each end sooner, until more waves only share a SIMD.
-// Lanes per wave 1 / 4 / 16 / 64, us: 1 000 sphere rays 42 / 41 / 48 / 52,
-// 8 000 point_in_volume 113 / 110 / 113 / 123, 100 000 sphere rays (25 at
-// least) 91 / 89 / 87 / 74.
-struct ResidentLaunch {
-  unsigned grid;
-  ResidentCfg c;
-  bool counted;  // some items are left for the shared counter
-};
-inline ResidentLaunch resident_launch(int64_t n, int64_t resident_blocks, int block, int refill, int min_lanes)
-{
-  const int64_t wpb = block / 64;
-  const int64_t waves = resident_blocks * wpb;
-  ResidentLaunch L;
-  const int64_t spread = std::max<int64_t>(1, waves / 4);
-  L.c.lanes_first = (int)std::min<int64_t>(64, (n + spread - 1) / spread);
-  const int64_t need = (n + L.c.lanes_first - 1) / L.c.lanes_first;  // waves
-  L.grid = (unsigned)std::min(resident_blocks, (need + wpb - 1) / wpb);
-  // eight ranges per wave keep the end of the launch balanced; 256 items
-  // amortise the atomic (chunk 64 / 256 / 512: 10 M nested-sphere rays
-  // 2.26 / 2.15 / 2.23 ms, 1 M sphere rays FP64 0.38 / 0.39 / 0.48 ms)
-  L.c.chunk = std::min<int64_t>(256, std::max<int64_t>(64, n / (waves * 8)));
-  L.c.refill = refill;
-  L.c.min_lanes = std::max(1, min_lanes * L.c.lanes_first / 64);
-  L.counted = (int64_t)L.grid * wpb * L.c.lanes_first < n;
-  return L;
 }
 
 #define XDG_DISPATCH2(KERNEL, MIXED, WIDE, ...)                                              \

@@ -298,6 +298,12 @@ __device__ inline D3 closest_on_triangle(const D3& v0, const D3& v1, const D3& v
 // plucker_tet_containment_test (src/tetrahedron_contain.cpp:11-43):
 // lambda123 = inverse(T) * (p - v0), T = [v1-v0, v2-v0, v3-v0] (columns);
 // inverse = adjugate / det (element-wise); lambda0 = 1 - (l1 + l2 + l3).
+// Most candidates are rejected before the nine divisions: with n_k the sum
+// whose terms the reference divides by det first, lambda_k differs from
+// n_k / det by a few units of 2^-53 of the terms' absolute sum m_k over
+// |det|, so n_k below -(tolerance + 2^-47 m_k) on det's scale puts lambda_k
+// below the tolerance (likewise lambda_0).  A zero or NaN det rejects
+// nothing here.
 __device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3& v1, const D3& v2, const D3& v3)
 {
   const D3 c0 = sub(v1, v0);
@@ -308,6 +314,19 @@ __device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3
   const D3 a1 = D3{c1.z * c2.x - c2.z * c1.x, c2.z * c0.x - c0.z * c2.x, c0.z * c1.x - c1.z * c0.x};
   const D3 a2 = D3{c1.x * c2.y - c2.x * c1.y, c2.x * c0.y - c0.x * c2.y, c0.x * c1.y - c1.x * c0.y};
   const double det = c0.x * a0.x + c0.y * a1.x + c0.z * a2.x;
+  const double hi = 1.0 + PLUCKER_ZERO_TOL;
+  {
+    const double sg = det < 0.0 ? -1.0 : 1.0, ad = fabs(det), tol = 2.0 * PLUCKER_ZERO_TOL * ad;
+    const double x1 = a0.x * r.x, y1 = a1.x * r.y, z1 = a2.x * r.z;
+    const double x2 = a0.y * r.x, y2 = a1.y * r.y, z2 = a2.y * r.z;
+    const double x3 = a0.z * r.x, y3 = a1.z * r.y, z3 = a2.z * r.z;
+    const double n1 = sg * (x1 + y1 + z1), n2 = sg * (x2 + y2 + z2), n3 = sg * (x3 + y3 + z3);
+    const double m1 = fabs(x1) + fabs(y1) + fabs(z1), m2 = fabs(x2) + fabs(y2) + fabs(z2),
+                 m3 = fabs(x3) + fabs(y3) + fabs(z3);
+    if (n1 < -(tol + 0x1p-47 * m1) || n2 < -(tol + 0x1p-47 * m2) || n3 < -(tol + 0x1p-47 * m3) ||
+        ad - (n1 + n2 + n3) < -(tol + 0x1p-47 * (m1 + m2 + m3 + ad)))
+      return false;
+  }
   const D3 i0 = D3{a0.x / det, a0.y / det, a0.z / det};
   const D3 i1 = D3{a1.x / det, a1.y / det, a1.z / det};
   const D3 i2 = D3{a2.x / det, a2.y / det, a2.z / det};
@@ -315,7 +334,6 @@ __device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3
   const double l2 = i0.y * r.x + i1.y * r.y + i2.y * r.z;
   const double l3 = i0.z * r.x + i1.z * r.y + i2.z * r.z;
   const double l0 = 1.0 - (l1 + l2 + l3);
-  const double hi = 1.0 + PLUCKER_ZERO_TOL;
   if (l0 < -PLUCKER_ZERO_TOL || l0 > hi) return false;
   if (l1 < -PLUCKER_ZERO_TOL || l1 > hi) return false;
   if (l2 < -PLUCKER_ZERO_TOL || l2 > hi) return false;
@@ -523,13 +541,12 @@ struct SurfTreeDev {
 };
 
 struct ElemTreeDev {
-  const NodeD* nodes_d;
-  const NodeF* nodes_f;
-  const int32_t* order;  // leaf-ordered element indices
+  const Node4F* nodes4_f;  // BVH4 over the elements' dilated boxes
+  const int32_t* order;    // leaf-ordered element indices
   const ElemRec* elems;
-  int32_t root;
+  int32_t root4;           // child-encoded root of the BVH4
   int32_t n_prims;
-  int32_t depth;
+  int32_t stack4;          // max traversal stack entries the BVH4 can need
   int32_t face_order[12];
   // implicit-complement re-entry (XDG::segments, xdg.cpp:164-185)
   int32_t ipc_tree;          // surface tree id, -1 if none
