@@ -126,10 +126,10 @@ int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent)
  *                 it starts new rays (1..64, default 32)
  *   "fv_refill"   the same for the persistent find_volume (1..64; 0, the
  *                 default: 24)
- *   "adjoint_sort" adjoint batches of >= 65536 rays with dldv: rays ordered
- *                 by hit face and each wave's run on one face summed before
- *                 the vertex atomics (1, default), or nine atomics per ray (0);
- *                 dldv's FP64 summation order differs, ray gradients do not
+ *   "adjoint_sort" adjoint batches of >= 65536 rays with dldv: each face's
+ *                 rays are summed before the vertex atomics (1, default), or
+ *                 nine atomics per ray (0); dldv's FP64 summation order
+ *                 differs, ray gradients do not
  *   "mw_wave"     mesh walk: particles that leave the mesh are parked and
  *                 their re-entry rays traced together in a separate kernel
  *                 (1), or each lane traces its own at once (0) (default 1)

@@ -1,0 +1,54 @@
+"""The binned adjoint (batches of at least 65 536 rays): meshes at the edges of
+a bucket of 256 faces, rays crowded on one face (several chunks of a bucket),
+a ragged last workgroup, hits without terms, and the largest bucket count
+beside the first mesh that falls back to the sorted form."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from gpu_util import bits, dev, host
+from xdg_amd import geometry as G
+from xdg_amd import philox as P
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from xdg_amd import capi
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("ntri,n,crowd", [(1, 65536, 0), (255, 65537, 0), (256, 70000, 0), (257, 65536, 0),
+                                          (1280, 100003, 40000), (1048320, 65536, 0), (1048321, 65536, 0)])
+def test_binned_adjoint(ctx, ntri, n, crowd):
+    m = G.perturbed_sphere(3, 10.0, 0.05)
+    reps = -(-ntri // m.tris.shape[0])
+    tris = np.ascontiguousarray(np.tile(m.tris, (reps, 1))[:ntri])
+    rng = np.random.default_rng(ntri + n)
+    face = rng.integers(0, ntri, n).astype(np.int32)
+    face[:crowd] = ntri // 2
+    b = rng.random((n, 2)) * 0.5
+    v = m.verts[tris[face]]
+    hit = v[:, 0] + b[:, :1] * (v[:, 1] - v[:, 0]) + b[:, 1:] * (v[:, 2] - v[:, 0])
+    org = P.ball_points(9, 0, n, 9.0)
+    t = np.linalg.norm(hit - org, axis=1)
+    dirs = (hit - org) / t[:, None]
+    w = rng.standard_normal(n)
+    face[::11] = -1
+    t[5::13] = np.inf
+    dirs[7::101] = 0.0  # no derivative: n.d = 0
+    face[3::503] = ntri + 5
+    gv = torch.zeros((m.verts.shape[0], 3), dtype=torch.float64, device="cuda")
+    go = torch.empty((n, 3), dtype=torch.float64, device="cuda")
+    gd = torch.empty_like(go)
+    ctx.ray_distance_adjoint(dev(torch, org), dev(torch, dirs), dev(torch, t), dev(torch, face), dev(torch, w),
+                             dev(torch, m.verts), dev(torch, tris), gv, go, gd)
+    ov, oo, od = O.adjoint(m.verts, tris, org, dirs, t, face, w)
+    assert np.array_equal(bits(host(go)), bits(oo)) and np.array_equal(bits(host(gd)), bits(od))
+    # at most n terms of the largest vertex sum's size, each rounded a few times
+    assert np.allclose(host(gv), ov, rtol=1e-12, atol=1e-12 * np.abs(ov).max())

@@ -121,6 +121,8 @@ struct xdg_hip_ctx {
   char* d_mw = nullptr;  // wavefront mesh walk scratch
   int64_t mw_cap = 0;
   MeshWalkScratch mw_w{};
+  void* d_adj = nullptr;  // binned adjoint: the rays' terms
+  int64_t adj_cap = 0;
   void* d_order = nullptr;  // ray ordering: keys, indices and sort storage
   int64_t order_cap = 0;
   RayOrderScratch order_w{};
@@ -362,6 +364,22 @@ const RayOrderScratch& order_scratch(xdg_hip_ctx* c, int64_t n)
   return c->order_w;
 }
 
+// the binned adjoint's memory for n rays (grown on demand, kept by the
+// context); null under capture when it would have to grow
+void* adjoint_scratch(xdg_hip_ctx* c, int64_t n, hipStream_t s)
+{
+  if (n > c->adj_cap) {
+    if (capturing(s)) return nullptr;
+    XDG_HIP_CHECK(hipDeviceSynchronize());
+    if (c->d_adj) XDG_HIP_CHECK(hipFree(c->d_adj));
+    c->d_adj = nullptr;
+    c->adj_cap = 0;
+    XDG_HIP_CHECK(hipMalloc(&c->d_adj, adjoint_bins_bytes(n)));
+    c->adj_cap = n;
+  }
+  return c->d_adj;
+}
+
 // the mixed kernels' deferral list, grown to n entries on demand
 int32_t* fb_list_for(xdg_hip_ctx* c, int64_t n)
 {
@@ -549,6 +567,7 @@ int xdg_hip_destroy(xdg_hip_ctx* c)
     if (c->d_fb_count) (void)hipFree(c->d_fb_count);
     if (c->d_next) (void)hipFree(c->d_next);
     if (c->d_order) (void)hipFree(c->d_order);
+    if (c->d_adj) (void)hipFree(c->d_adj);
     if (c->scratch_ev) (void)hipEventDestroy(c->scratch_ev);
     if (c->stream) (void)hipStreamDestroy(c->stream);
   }
@@ -1507,8 +1526,14 @@ int xdg_hip_ray_distance_adjoint(xdg_hip_ctx* c, int64_t n, const double* org, c
     if (!verts) a.ntri = 0;  // every ray reads as a miss without the mesh
     const hipStream_t s = pick(c, stream);
     if (c->cfg.adj_sort && dldv && n >= ORDER_MIN_RAYS) {
+      void* bins = nullptr;
+      const int nb = adjoint_buckets(a.ntri);
+      if (nb >= 1 && nb <= ADJ_BUCKETS_MAX && n < (int64_t)1 << 31) bins = adjoint_scratch(c, n, s);
       scratch_acquire(c, s);
-      launch_adjoint_sorted(a, order_scratch(c, n), s);
+      if (bins)
+        launch_adjoint_binned(a, bins, s);
+      else
+        launch_adjoint_sorted(a, order_scratch(c, n), s);
       XDG_HIP_CHECK(hipGetLastError());
       scratch_release(c, s);
     } else {

@@ -378,6 +378,23 @@ void launch_adjoint(const AdjointArgs& a, int block, hipStream_t s);
 // at least a.n entries); the vertex sums run per wave and face
 void launch_adjoint_sorted(const AdjointArgs& a, const RayOrderScratch& w, hipStream_t s);
 
+// the binned form: rays' terms in buckets of faces (see adjoint.hip), for
+// meshes of at most ADJ_BUCKETS_MAX buckets; mem holds
+// adjoint_bins_bytes(a.n) bytes, 256-byte aligned
+constexpr int ADJ_BUCKETS_MAX = 4095;  // and a total: 4096 entries
+struct alignas(16) AdjointEntry {
+  double w, x, y, z;
+};
+struct AdjointBins {
+  int nb;
+  AdjointEntry* terms;
+  uint8_t* local;  // face within its bucket
+  uint32_t *cnt, *cur, *off, *chunk;
+};
+int adjoint_buckets(int64_t ntri);
+size_t adjoint_bins_bytes(int64_t n);
+void launch_adjoint_binned(const AdjointArgs& a, void* mem, hipStream_t s);
+
 // ---- element queries (element_query.hip) ---------------------------------
 struct FindElementArgs {
   const xdgd::ElemTreeDev* etable;
