@@ -109,3 +109,21 @@ def test_find_element_split(setup, n):
     assert np.array_equal(got[:k], om.find_element(p[:k]))
     for lo in range(k, n, 50000):
         assert np.array_equal(got[lo:lo + 50000], host(ctx.find_element(et, dev(torch, p[lo:lo + 50000]))))
+
+
+def test_segments_ending_on_the_boundary(setup):
+    """Segments whose ends are clamped onto the mesh's faces, edges and
+    corners: some come round the segment loop without moving, up to its cap."""
+    import pyoracle as O
+    ctx = setup[0]
+    mesh = G.kuhn_cube(9, 0.2, seed=4)
+    et = ctx.build_element_tree(mesh.verts, mesh.tets, mesh.adj, mesh.face_order)
+    bm = mesh.boundary_model()
+    ctx.attach_boundary(et, build_tree(ctx, bm, bm.ipc), mesh.bface_elem)
+    n = 60000
+    p0 = P.box_points(75, P.STREAM_POS, n, [0.0] * 3, [1.0] * 3)
+    p1 = np.clip(p0 + P.iso_dirs(75, P.STREAM_DIR, n) * np.geomspace(1e-3, 2.0, n)[:, None], 0.0, 1.0)
+    tally = torch.zeros(mesh.tets.shape[0], dtype=torch.int64, device="cuda")
+    cnt, hsh = [host(x) for x in ctx.tally_segments(et, dev(torch, p0), dev(torch, p1), tally=tally)]
+    rc, rh = O.TetMesh(mesh).segments(p0, p1)
+    assert np.array_equal(cnt, rc) and np.array_equal(hsh.view(np.uint64), rh)

@@ -513,12 +513,20 @@ __global__ void k_segments(SegmentsArgs a, int cap)
   int32_t last = ID_NONE;
   int steps = 0, loops = 0;
   bool capped = false;
+  // A segment that ends on the mesh's boundary may come round here without
+  // having moved, up to the loop cap.  The element at an unchanged position
+  // is the one found before: 64 point locations of one lane took half of a
+  // launch (200 001 short segments, 32^3 x 6 tets: 1.21 -> 0.71 ms).
+  bool moved = true;
+  int32_t found = ID_NONE;
   while (distance > 0) {
     if (++loops > MAX_SEG_LOOPS || steps >= MAX_WALK_STEPS) {
       capped = true;
       break;
     }
-    int32_t cur = find_element_dev(T, r, stk, stride);
+    if (moved) found = find_element_dev(T, r, stk, stride);
+    const D3 at = r;
+    int32_t cur = found;
     if (s.count > 0 && cur == last) cur = ID_NONE;
     if (cur == ID_NONE) {
       // xdg.cpp:164-185: fire against the implicit complement
@@ -558,6 +566,7 @@ __global__ void k_segments(SegmentsArgs a, int cap)
     r.y = r.y + sum * u.y;
     r.z = r.z + sum * u.z;
     distance -= sum;
+    moved = !(r.x == at.x && r.y == at.y && r.z == at.z);
   }
   a.count[i] = s.count;
   a.hash[i] = s.hash;
