@@ -138,9 +138,10 @@ __device__ __forceinline__ void write_hit(const RayFireArgs& a, int64_t i, const
 // 0.456 -> 0.383 ms: ranges per wave instead of one atomic per refill,
 // leaving the node loop when few lanes descend, pushes without branches
 // (wave instructions 110 -> 88 per ray, active lanes 27 -> 37 %).
-template <bool MIXED>
+// FEW: a far-origin ray is traced with FP64 boxes at once instead.
+template <bool MIXED, bool FEW = false>
 __device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, unsigned long long* next_ray,
-                                                 const ResidentCfg& c)
+                                                 const ResidentCfg& c, int cap = 0)
 {
   extern __shared__ int32_t lds[];
   GuardedStack S(lds + threadIdx.x, blockDim.x);
@@ -181,10 +182,13 @@ __device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, unsigned 
         if (tree >= 1 && tree <= a.ntrees) {
           const SurfTreeDev& TT = a.table[tree];
           ray = make_ray(a.org + 3 * ri, a.dir + 3 * ri);
-          if (MIXED && !mixed_safe(TT, ray)) {
+          if (MIXED && !FEW && !mixed_safe(TT, ray)) {
             const unsigned int j = atomicAdd(a.fb_count, 1u);
             a.fb_list[j] = (int32_t)ri;
             have = false;
+          } else if (MIXED && FEW && !mixed_safe(TT, ray)) {
+            traverse4<RAYFIRE, false>(TT, ray, a.orientation, a.excl ? a.excl + (int64_t)a.k * ri : nullptr, k, S.base,
+                                      S.stride, cap, h);
           } else {
             T.nodes4_d = TT.nodes4_d;
             T.nodes4_f = TT.nodes4_f;
@@ -213,6 +217,14 @@ __device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, unsigned 
 __global__ void k_ray_fire_pt_mixed(RayFireArgs a, unsigned long long* next_ray, ResidentCfg c)
 {
   ray_fire_pt_body<true>(a, next_ray, c);
+}
+// Mixed batches that leave every wave with fewer than 64 rays: no counter, no
+// deferral list, and so one launch instead of three (1 000 rays: 41 -> 37
+// us a call).  The FP64 boxes' state costs registers, which larger batches
+// would pay for in waves per SIMD.
+__global__ __launch_bounds__(256) void k_ray_fire_few_mixed(RayFireArgs a, ResidentCfg c, int cap)
+{
+  ray_fire_pt_body<true, true>(a, nullptr, c, cap);
 }
 __global__ void k_ray_fire_pt_plain(RayFireArgs a, unsigned long long* next_ray, ResidentCfg c)
 {
@@ -899,6 +911,10 @@ void launch_ray_fire(const RayFireArgs& a, bool mixed, const LaunchCfg& c, hipSt
     const ResidentLaunch L =
         resident_launch(a.n, mixed ? resident_grid(k_ray_fire_pt_mixed, c.block, shg)
                                    : resident_grid(k_ray_fire_pt_plain, c.block, shg), c.block, c.refill, RF_MIN_LANES);
+    if (mixed && !L.counted && L.c.lanes_first < 64 && c.block <= 256) {
+      hipLaunchKernelGGL(k_ray_fire_few_mixed, dim3(L.grid), b, shg, s, a, L.c, c.stack);
+      return;
+    }
     if (mixed || L.counted)
       hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(1), 0, s, a.next_ray, mixed ? a.fb_count : nullptr);
     if (mixed) {
