@@ -1779,7 +1779,7 @@ int xdg_hip_transport_create(xdg_hip_ctx* c, const xdg_hip_transport_problem* p,
       }
       t->d_next = (unsigned long long*)dev_alloc(64, t->bufs);
       t->d_live = (uint32_t*)dev_alloc(64, t->bufs);
-      t->dev.pre_box = (double*)dev_alloc((size_t)p->nvol * 6 * sizeof(double), t->bufs);
+      t->dev.pre_box = (float*)dev_alloc((size_t)p->nvol * 6 * sizeof(float), t->bufs);
       t->dev.slot_cnt = (uint32_t*)dev_alloc(((size_t)p->nvol + 1) * sizeof(uint32_t), t->bufs);
       t->dev.slot_cur = (uint32_t*)dev_alloc((size_t)p->nvol * sizeof(uint32_t), t->bufs);
       t->host_trees.assign(p->vol_trees, p->vol_trees + p->nvol);

@@ -281,7 +281,7 @@ struct TransportDev {
   double mfp, p_absorb;
   int32_t max_events;
   const uint8_t* surf_bc;   // nullable: boundary condition per surface id [0, nsurf)
-  double* pre_box;          // nvol x (lo.xyz, hi.xyz): start-stage prefilter boxes, written per launch
+  float* pre_box;           // nvol x (lo.xyz, hi.xyz): start-stage prefilter boxes, written per launch
   uint32_t* slot_cnt;       // nvol + 1: start-stage items per volume slot, then their offsets (+ total)
   uint32_t* slot_cur;       // nvol: scatter cursors
 };
