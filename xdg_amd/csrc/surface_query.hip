@@ -205,10 +205,8 @@ __device__ __forceinline__ void ray_fire_pt_body(const RayFireArgs& a, unsigned 
     }
     descend4<MIXED>(T, S, bf, bd, po, tf, h.t, c.min_lanes, node, leaf);
     if (leaf != DONE) {
-      const int32_t first = leaf_first(leaf);
-      const int32_t cnt = leaf_count(leaf);
+      leaf_pairs<RAYFIRE>(T, leaf, ray, a.orientation, ex, k, h);
       leaf = DONE;
-      for (int32_t j = 0; j < cnt; ++j) tri_closest_hit<RAYFIRE>(T, first + j, ray, a.orientation, ex, k, h);
       tf = f32_up(h.t);
     }
   }
@@ -357,10 +355,8 @@ __device__ __forceinline__ void piv_pt_body(const PivArgs& a, int cap, const Res
     }
     descend4<MIXED>(T, S, bf, bd, po, tf, h.t, c.min_lanes, node, leaf);
     if (leaf != DONE) {
-      const int32_t first = leaf_first(leaf);
-      const int32_t cnt = leaf_count(leaf);
+      leaf_pairs<PIV>(T, leaf, ray, ORIENT_ANY, ex, k, h);
       leaf = DONE;
-      for (int32_t j = 0; j < cnt; ++j) tri_closest_hit<PIV>(T, first + j, ray, ORIENT_ANY, ex, k, h);
       tf = f32_up(h.t);
     }
   }
