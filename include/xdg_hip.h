@@ -19,8 +19,9 @@
  *   - Calls on one context from several host threads are serialized.
  *   - Streams: queries on different streams may overlap, except that the
  *     context's shared scratch (the persistent kernels' work counters, the
- *     mixed-precision deferral list, the ray-ordering buffers, the mesh
- *     walk's particle store) serves one launch at a time.  The library
+ *     mixed-precision deferral list, the ray-ordering buffers, the
+ *     adjoint's bins, the mesh walk's particle store) serves one launch at
+ *     a time.  The library
  *     orders those launches itself: a ray_fire, find_volume or wavefront
  *     mesh walk on stream B waits (hipStreamWaitEvent) for the last such
  *     launch on stream A.  Under graph capture that ordering is the
