@@ -127,3 +127,25 @@ def test_segments_ending_on_the_boundary(setup):
     cnt, hsh = [host(x) for x in ctx.tally_segments(et, dev(torch, p0), dev(torch, p1), tally=tally)]
     rc, rh = O.TetMesh(mesh).segments(p0, p1)
     assert np.array_equal(cnt, rc) and np.array_equal(hsh.view(np.uint64), rh)
+
+
+@pytest.mark.parametrize("jitter", [0.0, 0.2])
+@pytest.mark.parametrize("m", [1, 3, 4, 7])
+def test_element_records(setup, m, jitter):
+    """Trees of fewer elements than a block, ragged and several blocks of the
+    record kernel; without jitter, edges whose ends tie in x and y.  The walks
+    use every field of the records and equal the oracle."""
+    import pyoracle as O
+    ctx = setup[0]
+    mesh = G.kuhn_cube(m, jitter, seed=4)
+    et = ctx.build_element_tree(mesh.verts, mesh.tets, mesh.adj, mesh.face_order)
+    bm = mesh.boundary_model()
+    ctx.attach_boundary(et, build_tree(ctx, bm, bm.ipc), mesh.bface_elem)
+    n = 3000
+    p0 = P.box_points(77, P.STREAM_POS, n, [-0.2] * 3, [1.2] * 3)
+    p1 = p0 + P.iso_dirs(77, P.STREAM_DIR, n)
+    om = O.TetMesh(mesh)
+    assert np.array_equal(host(ctx.find_element(et, dev(torch, p0))), om.find_element(p0))
+    cnt, hsh = [host(x) for x in ctx.tally_segments(et, dev(torch, p0), dev(torch, p1))]
+    rc, rh = om.segments(p0, p1)
+    assert np.array_equal(cnt, rc) and np.array_equal(hsh.view(np.uint64), rh)

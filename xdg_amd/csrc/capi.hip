@@ -822,27 +822,9 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
     if (face_order) {
       for (int f = 0; f < 12; ++f) require(face_order[f] >= 0 && face_order[f] < 4, "face_order entries must be 0..3");
     }
-    std::vector<ElemRec> recs((size_t)n_tets);
-    for (int64_t e = 0; e < n_tets; ++e) {
-      ElemRec& r = recs[e];
-      for (int j = 0; j < 4; ++j) {
-        int32_t vi = tets[4 * e + j];
-        require(vi >= 0 && vi < n_verts, "tet vertex index out of range");
-        if (j < 3) r.conn[j] = vi;
-        for (int k = 0; k < 3; ++k) r.v[3 * j + k] = verts[3 * (int64_t)vi + k];
-        int32_t a = adj[4 * e + j];
-        require(a >= -1 && a < n_tets, "adjacency out of range");
-        r.adj[j] = a;
-      }
-      // lexicographic endpoint order of the six edges (plucker.h:35-43)
-      static const int pa[6] = {0, 0, 0, 1, 1, 2}, pb[6] = {1, 2, 3, 2, 3, 3};
-      r.edge_first = 0;
-      for (int k = 0; k < 6; ++k) {
-        const double* a = r.v + 3 * pa[k];
-        const double* b = r.v + 3 * pb[k];
-        const bool f = a[0] < b[0] || (!(a[0] > b[0]) && (a[1] < b[1] || (!(a[1] > b[1]) && a[2] < b[2])));
-        r.edge_first |= (f ? 1u : 0u) << k;
-      }
+    for (int64_t k = 0; k < 4 * n_tets; ++k) {
+      require(tets[k] >= 0 && tets[k] < n_verts, "tet vertex index out of range");
+      require(adj[k] >= -1 && adj[k] < n_tets, "adjacency out of range");
     }
     hipStream_t s = c->stream;
     ElemTreeHost t;
@@ -851,8 +833,17 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
       size_t ne = (size_t)std::max<int64_t>(n_tets, 1);
       ElemRec* d_elems = (ElemRec*)dev_alloc(ne * sizeof(ElemRec), t.bufs);
       double* d_box = (double*)dev_alloc(ne * 6 * sizeof(double), tmp);
-      if (n_tets > 0)
-        XDG_HIP_CHECK(hipMemcpyAsync(d_elems, recs.data(), (size_t)n_tets * sizeof(ElemRec), hipMemcpyHostToDevice, s));
+      if (n_tets > 0) {
+        // the mesh's own arrays go up (a quarter of the records' bytes) and
+        // the records are written on the device
+        const size_t vb = sizeof(double) * 3 * (size_t)n_verts, tb = sizeof(int32_t) * 4 * (size_t)n_tets;
+        char* d_in = (char*)dev_alloc(vb + 2 * tb, tmp);
+        XDG_HIP_CHECK(hipMemcpyAsync(d_in, verts, vb, hipMemcpyHostToDevice, s));
+        XDG_HIP_CHECK(hipMemcpyAsync(d_in + vb, tets, tb, hipMemcpyHostToDevice, s));
+        XDG_HIP_CHECK(hipMemcpyAsync(d_in + vb + tb, adj, tb, hipMemcpyHostToDevice, s));
+        launch_elem_records((const double*)d_in, (const int32_t*)(d_in + vb), (const int32_t*)(d_in + vb + tb), n_tets,
+                            d_elems, s);
+      }
       launch_elem_boxes(d_elems, n_tets, d_box, s);
       LbvhOut lb;
       lbvh_build(d_box, n_tets, c->leaf_max, s, t.bufs, lb, false, c->build_sah != 0);

