@@ -1,0 +1,111 @@
+// CPU checks of xdg_amd/csrc/fp32_bounds.h, the conservative FP32 tests of
+// the kernels (host side of the same functions).  argv[1] names the check;
+// prints "ok" or what failed.
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <random>
+
+#include "fp32_bounds.h"
+
+using namespace xdgd;
+
+namespace {
+
+std::mt19937_64 rng(12345);
+double uni() { return std::uniform_real_distribution<double>(0.0, 1.0)(rng); }
+double nrm() { return std::normal_distribution<double>()(rng); }
+
+typedef long double LD;
+struct L3 {
+  LD x, y, z;
+};
+L3 l3(const D3& a) { return L3{a.x, a.y, a.z}; }
+L3 operator-(const L3& a, const L3& b) { return L3{a.x - b.x, a.y - b.y, a.z - b.z}; }
+LD dotl(const L3& a, const L3& b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+L3 crossl(const L3& a, const L3& b)
+{
+  return L3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+}
+
+LD segment_distance(const L3& p, const L3& a, const L3& e)
+{
+  const L3 w = p - a;
+  const LD ee = dotl(e, e);
+  LD s = ee > 0 ? dotl(w, e) / ee : 0;
+  s = s < 0 ? 0 : (s > 1 ? 1 : s);
+  const L3 d{w.x - s * e.x, w.y - s * e.y, w.z - s * e.z};
+  return sqrtl(dotl(d, d));
+}
+
+// distance of p to the triangle in 80-bit arithmetic
+LD distance(const D3& v0, const D3& v1, const D3& v2, const D3& q)
+{
+  const L3 a = l3(v0), p = l3(q), e0 = l3(v1) - a, e1 = l3(v2) - a, e2 = e1 - e0, w = p - a;
+  LD best = fminl(fminl(segment_distance(p, a, e0), segment_distance(p, a, e1)), segment_distance(p, l3(v1), e2));
+  const L3 n = crossl(e0, e1);
+  const LD nn = dotl(n, n);
+  if (nn > 0) {
+    const LD u = dotl(crossl(w, e1), n) / nn, v = dotl(crossl(e0, w), n) / nn;
+    if (u >= 0 && v >= 0 && u + v <= 1) best = fminl(best, fabsl(dotl(w, n)) / sqrtl(nn));
+  }
+  return best;
+}
+
+// the normal as the tree stores it (face_normal's operations)
+D3 normal(const D3& v0, const D3& v1, const D3& v2)
+{
+  D3 n = cross(sub(v1, v0), sub(v2, v0));
+  double len = sqrt(n.x * n.x + n.y * n.y + n.z * n.z);
+  len = len < (double)MIN_RCP_INPUT ? (double)MIN_RCP_INPUT : len;
+  return D3{n.x / len, n.y / len, n.z / len};
+}
+
+D3 rnd(double s) { return D3{s * nrm(), s * nrm(), s * nrm()}; }
+
+// closest_beyond keeps every triangle whose distance is the best one, with
+// points near to and far from it, everything scaled by 10^e for e in
+// [lo, hi].  thin: aspects down to 1e-16.
+int closest_bound(int lo, int hi, bool thin)
+{
+  long wrong = 0, rejected = 0, total = 0;
+  for (int e = lo; e <= hi; ++e) {
+    const double scale = std::pow(10.0, e);
+    long w = 0;
+    for (int k = 0; k < 20000; ++k) {
+      const double size = std::pow(10.0, -3.0 * uni());
+      const double aspect = thin ? std::pow(10.0, -16.0 * uni()) : 1.0, f = 2.0 * uni() - 0.5;
+      const D3 d1 = rnd(size), off = rnd(size * aspect);
+      D3 v0 = rnd(k % 2 ? 1.0 : 0.0), v1{v0.x + d1.x, v0.y + d1.y, v0.z + d1.z};
+      D3 v2{v0.x + f * d1.x + off.x, v0.y + f * d1.y + off.y, v0.z + f * d1.z + off.z};
+      const double b = 1.4 * uni() - 0.2, c = 1.4 * uni() - 0.2, h = size * std::pow(10.0, 1.0 - 4.0 * uni());
+      const D3 dn = k % 4 < 2 ? normal(v0, v1, v2) : rnd(1.0);
+      D3 p{v0.x + b * (v1.x - v0.x) + c * (v2.x - v0.x) + h * dn.x,
+           v0.y + b * (v1.y - v0.y) + c * (v2.y - v0.y) + h * dn.y,
+           v0.z + b * (v1.z - v0.z) + c * (v2.z - v0.z) + h * dn.z};
+      for (D3* q : {&v0, &v1, &v2, &p}) *q = D3{q->x * scale, q->y * scale, q->z * scale};
+      const D3 n = normal(v0, v1, v2);
+      const double d = (double)distance(v0, v1, v2, p);
+      w += closest_beyond(v0, v1, v2, n, p, f32_up(d * d));
+      rejected += closest_beyond(v0, v1, v2, n, p, f32_up(0.49 * d * d));
+      ++total;
+    }
+    if (w) std::printf("scale 1e%d: %ld of 20000 triangles at the best distance rejected\n", e, w);
+    wrong += w;
+  }
+  if (rejected * 4 < 20000) {
+    std::printf("only %ld of %ld farther triangles rejected\n", rejected, total);
+    ++wrong;
+  }
+  return wrong != 0;
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+  int rc = 1;
+  if (argc == 2 && !std::strcmp(argv[1], "closest")) rc = closest_bound(-24, 24, false);
+  if (!rc) std::printf("ok\n");
+  return rc;
+}

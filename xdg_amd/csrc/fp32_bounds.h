@@ -1,0 +1,81 @@
+// fp32_bounds.h -- FP32 tests that decide which candidates get the FP64
+// arithmetic: rounding helpers and conservative bounds.  Host and device, so
+// that CPU tests compile the code the kernels run.
+#pragma once
+
+#include "xdg_device.h"
+
+namespace xdgd {
+
+__host__ __device__ __forceinline__ float safe_inv_f(float d)
+{
+  const float eps = 1e-30f;
+  return 1.0f / (fabsf(d) > eps ? d : copysignf(eps, d));
+}
+
+__host__ __device__ __forceinline__ float f32_up(double x)
+{
+  float f = (float)x;
+  if ((double)f < x) f = nextafterf(f, INFINITY);
+  return f;
+}
+__host__ __device__ __forceinline__ float f32_down_d(double x)
+{
+  float f = (float)x;
+  if ((double)f > x) f = nextafterf(f, -INFINITY);
+  return f;
+}
+
+// 1/x within two units in the last place; the host's is the correctly rounded
+// one
+__host__ __device__ __forceinline__ float rcp_approx(float x)
+{
+#if __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcpf(x);
+#else
+  return 1.0f / x;
+#endif
+}
+
+// Is the triangle certainly farther from p than best?  An FP32 distance to
+// its three edges, or to its plane (FP64, stored normal) where p projects
+// inside it, against best^2.  With M the sum of squares of p - v0 and two
+// edges, every FP32 quantity here is off by at most about 10 x 2^-24 M; a
+// projection misjudged as outside lies within 4 x 2^-24 M (squared) of an
+// edge whatever the triangle's shape, and the plane is never farther than
+// the triangle.  The margin is 2^-17 M.  The products of four lengths leave
+// FP32's normal range for M above 2^64 or well below 2^-50 (projections are
+// then misjudged by more than that): the test rejects nothing there, nor
+// where a coordinate is NaN.
+// Box distances let about 100 triangles per point pass on a sphere of
+// 20 480 (an inclined triangle's box reaches far beyond it) of which a few
+// need the FP64 closest point, four times this test's work.
+__host__ __device__ __forceinline__ bool closest_beyond(const D3& v0, const D3& v1, const D3& v2, const D3& n,
+                                                        const D3& p, float best2)
+{
+  const D3 d0 = sub(v0, p), d1 = sub(v1, v0), d2 = sub(v2, v0);
+  const double plane = n.x * d0.x + n.y * d0.y + n.z * d0.z;
+  const float wx = (float)d0.x, wy = (float)d0.y, wz = (float)d0.z;
+  const float sx = (float)d1.x, sy = (float)d1.y, sz = (float)d1.z;
+  const float tx = (float)d2.x, ty = (float)d2.y, tz = (float)d2.z;
+  const float pp = wx * wx + wy * wy + wz * wz;
+  const float ss = sx * sx + sy * sy + sz * sz;
+  const float tt = tx * tx + ty * ty + tz * tz;
+  const float m = pp + ss + tt;
+  const float st = sx * tx + sy * ty + sz * tz;
+  const float sp = sx * wx + sy * wy + sz * wz;
+  const float tp = tx * wx + ty * wy + tz * wz;
+  const float s = st * tp - tt * sp, t = st * sp - ss * tp;
+  const bool inside = s >= 0.0f && t >= 0.0f && s + t <= ss * tt - st * st;
+  // edges v0v1, v0v2 and v1v2: |w + a e|^2 at the clamped minimum
+  const float a = fminf(fmaxf(-sp * rcp_approx(ss), 0.0f), 1.0f);
+  const float b = fminf(fmaxf(-tp * rcp_approx(tt), 0.0f), 1.0f);
+  const float ee = ss - 2.0f * st + tt, qe = (tp - sp) + (st - ss), qq = pp + 2.0f * sp + ss;
+  const float c = fminf(fmaxf(-qe * rcp_approx(ee), 0.0f), 1.0f);
+  const float e0 = pp + a * (2.0f * sp + a * ss), e1 = pp + b * (2.0f * tp + b * tt), e2 = qq + c * (2.0f * qe + c * ee);
+  const float pl = (float)plane;
+  const float lb = inside ? pl * pl : fminf(fminf(e0, e1), e2);
+  return m >= 0x1p-50f && m <= 0x1p60f && lb - 0x1p-17f * m > best2;
+}
+
+}  // namespace xdgd

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cstddef>
 
+#include "fp32_bounds.h"
 #include "internal.h"
 #include "surface_traverse.h"
 #include "xdg_hip.h"
@@ -552,43 +553,6 @@ __device__ __forceinline__ double box_d2(const double* b, const D3& p)
   double ey = fmax(fmax(b[1] - p.y, p.y - b[4]), 0.0);
   double ez = fmax(fmax(b[2] - p.z, p.z - b[5]), 0.0);
   return ex * ex + ey * ey + ez * ez;
-}
-
-// Is the triangle certainly farther from p than best?  An FP32 distance to
-// its three edges, or to its plane (FP64, stored normal) where p projects
-// inside it, against best^2.  With M the sum of squares of p - v0 and two
-// edges, every FP32 quantity here is off by at most about 10 x 2^-24 M; a
-// projection misjudged as outside lies within 4 x 2^-24 M (squared) of an
-// edge whatever the triangle's shape, and the plane is never farther than
-// the triangle.  The margin is 2^-17 M.  NaN (overflow) answers no.
-// Box distances let about 100 triangles per point pass on a sphere of
-// 20 480 (an inclined triangle's box reaches far beyond it) of which a few
-// need the FP64 closest point, four times this test's work.
-__device__ __forceinline__ bool closest_beyond(const D3& v0, const D3& v1, const D3& v2, const D3& n, const D3& p,
-                                               float best2)
-{
-  const D3 d0 = sub(v0, p), d1 = sub(v1, v0), d2 = sub(v2, v0);
-  const double plane = n.x * d0.x + n.y * d0.y + n.z * d0.z;
-  const float wx = (float)d0.x, wy = (float)d0.y, wz = (float)d0.z;
-  const float sx = (float)d1.x, sy = (float)d1.y, sz = (float)d1.z;
-  const float tx = (float)d2.x, ty = (float)d2.y, tz = (float)d2.z;
-  const float pp = wx * wx + wy * wy + wz * wz;
-  const float ss = sx * sx + sy * sy + sz * sz;
-  const float tt = tx * tx + ty * ty + tz * tz;
-  const float st = sx * tx + sy * ty + sz * tz;
-  const float sp = sx * wx + sy * wy + sz * wz;
-  const float tp = tx * wx + ty * wy + tz * wz;
-  const float s = st * tp - tt * sp, t = st * sp - ss * tp;
-  const bool inside = s >= 0.0f && t >= 0.0f && s + t <= ss * tt - st * st;
-  // edges v0v1, v0v2 and v1v2: |w + a e|^2 at the clamped minimum
-  const float a = fminf(fmaxf(-sp * __builtin_amdgcn_rcpf(ss), 0.0f), 1.0f);
-  const float b = fminf(fmaxf(-tp * __builtin_amdgcn_rcpf(tt), 0.0f), 1.0f);
-  const float ee = ss - 2.0f * st + tt, qe = (tp - sp) + (st - ss), qq = pp + 2.0f * sp + ss;
-  const float c = fminf(fmaxf(-qe * __builtin_amdgcn_rcpf(ee), 0.0f), 1.0f);
-  const float e0 = pp + a * (2.0f * sp + a * ss), e1 = pp + b * (2.0f * tp + b * tt), e2 = qq + c * (2.0f * qe + c * ee);
-  const float pl = (float)plane;
-  const float lb = inside ? pl * pl : fminf(fminf(e0, e1), e2);
-  return lb - 0x1p-17f * (pp + ss + tt) > best2;
 }
 
 // The triangles of one leaf against the best distance and face so far (ties:

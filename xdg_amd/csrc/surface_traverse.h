@@ -5,6 +5,7 @@
 // surface_query.hip for the semantics and the tie rule.
 #pragma once
 
+#include "fp32_bounds.h"
 #include "xdg_device.h"
 
 namespace xdgd {
@@ -29,25 +30,6 @@ __device__ __forceinline__ double safe_inv_d(double d)
   const double eps = 1e-300;
   return 1.0 / (fabs(d) > eps ? d : copysign(eps, d));
 }
-__device__ __forceinline__ float safe_inv_f(float d)
-{
-  const float eps = 1e-30f;
-  return 1.0f / (fabsf(d) > eps ? d : copysignf(eps, d));
-}
-
-__device__ __forceinline__ float f32_up(double x)
-{
-  float f = (float)x;
-  if ((double)f < x) f = nextafterf(f, INFINITY);
-  return f;
-}
-__device__ __forceinline__ float f32_down_d(double x)
-{
-  float f = (float)x;
-  if ((double)f > x) f = nextafterf(f, -INFINITY);
-  return f;
-}
-
 // slab test of one box; returns entry distance in tn
 __device__ __forceinline__ bool slab_d(const double* b, const BoxRayD& r, double tmax, double& tn)
 {
