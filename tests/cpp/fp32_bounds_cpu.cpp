@@ -106,6 +106,7 @@ int main(int argc, char** argv)
 {
   int rc = 1;
   if (argc == 2 && !std::strcmp(argv[1], "closest")) rc = closest_bound(-24, 24, false);
+  if (argc == 2 && !std::strcmp(argv[1], "closest_thin")) rc = closest_bound(-24, 24, true);
   if (!rc) std::printf("ok\n");
   return rc;
 }

@@ -21,9 +21,9 @@ def ctx():
     c.close()
 
 
-def check(ctx, v9, bump, pts):
+def check(ctx, v9, bump, pts, face=None):
     n = len(v9)
-    face = np.arange(n, dtype=np.int32)
+    face = np.arange(n, dtype=np.int32) if face is None else face
     surf, flip = np.ones(n, np.int32), np.zeros(n, np.uint8)
     tree = ctx.build_surface_tree(v9.reshape(-1, 3), np.arange(3 * n, dtype=np.int32).reshape(-1, 3), face, surf,
                                   flip, bump)
@@ -40,3 +40,19 @@ def test_closest_scales(ctx, radius, subdiv):
     v, t = G.icosphere(subdiv, radius)
     pts = P.ball_points(81, 0, 2000, 1.5 * radius)
     check(ctx, v[t].reshape(-1, 9), 1e-6 * radius, pts)
+
+
+def test_closest_thin_triangles(ctx):
+    """Triangles of aspects down to 1e-16, whose stored normals are far from
+    exact, each twice with the lower face id second: the second must not be
+    rejected at the best distance."""
+    rng = np.random.default_rng(83)
+    n = 4000
+    v0, d1 = rng.standard_normal((n, 3)), rng.standard_normal((n, 3)) * 0.05
+    off = rng.standard_normal((n, 3)) * 0.05 * 10.0 ** rng.uniform(-16, 0, (n, 1))
+    v9 = np.hstack([v0, v0 + d1, v0 + rng.uniform(-0.5, 1.5, (n, 1)) * d1 + off])
+    v9 = np.repeat(v9, 2, axis=0)
+    b = rng.random((20 * n, 1))
+    pts = np.repeat(v0, 20, axis=0) + b * np.repeat(d1, 20, axis=0)
+    pts = pts + rng.standard_normal(pts.shape) * 0.05 * 10.0 ** rng.uniform(-3, 0, (20 * n, 1))
+    check(ctx, v9, 1e-9, pts, np.arange(2 * n, dtype=np.int32)[::-1].copy())

@@ -43,7 +43,10 @@ __host__ __device__ __forceinline__ float rcp_approx(float x)
 // edges, every FP32 quantity here is off by at most about 10 x 2^-24 M; a
 // projection misjudged as outside lies within 4 x 2^-24 M (squared) of an
 // edge whatever the triangle's shape, and the plane is never farther than
-// the triangle.  The margin is 2^-17 M.  The products of four lengths leave
+// the triangle.  A triangle thinner than 2^-10 of its length goes by its
+// edges alone, which are within 2^-20 M (squared) of its interior: FP32 does
+// not tell inside from outside there, and the stored normal of a far thinner
+// one is off by more than the margin.  The margin is 2^-17 M.  The products of four lengths leave
 // FP32's normal range for M above 2^64 or well below 2^-50 (projections are
 // then misjudged by more than that): the test rejects nothing there, nor
 // where a coordinate is NaN.
@@ -66,7 +69,8 @@ __host__ __device__ __forceinline__ bool closest_beyond(const D3& v0, const D3& 
   const float sp = sx * wx + sy * wy + sz * wz;
   const float tp = tx * wx + ty * wy + tz * wz;
   const float s = st * tp - tt * sp, t = st * sp - ss * tp;
-  const bool inside = s >= 0.0f && t >= 0.0f && s + t <= ss * tt - st * st;
+  const float pr = ss * tt, det = pr - st * st;
+  const bool inside = s >= 0.0f && t >= 0.0f && s + t <= det && det > 0x1p-20f * pr;
   // edges v0v1, v0v2 and v1v2: |w + a e|^2 at the clamped minimum
   const float a = fminf(fmaxf(-sp * rcp_approx(ss), 0.0f), 1.0f);
   const float b = fminf(fmaxf(-tp * rcp_approx(tt), 0.0f), 1.0f);
