@@ -100,6 +100,48 @@ int closest_bound(int lo, int hi, bool thin)
   return wrong != 0;
 }
 
+// a box whose vertices' bounds are at the best distance or nearer passes the
+// limit, at every scale whose distances' squares FP64 holds exactly enough
+int closest_boxes()
+{
+  long wrong = 0, passed = 0, total = 0;
+  for (int e = -44; e <= 18; ++e) {
+    const double scale = std::pow(10.0, e);
+    long w = 0;
+    for (int k = 0; k < 20000; ++k) {
+      const double bump = scale * std::pow(10.0, -2.0 - 12.0 * uni());
+      double lo[3], hi[3], q[3], ext = 0.0;
+      float flo[3], fhi[3];
+      for (int j = 0; j < 3; ++j) {
+        lo[j] = scale * nrm();
+        hi[j] = lo[j] + scale * uni();
+        q[j] = scale * 2.0 * nrm();
+        ext = std::fmax(ext, std::fmax(std::fabs(lo[j]), std::fabs(hi[j])) + bump);
+        flo[j] = f32_down_d(lo[j] - bump);
+        fhi[j] = f32_up(hi[j] + bump);
+      }
+      LD d2 = 0;
+      for (int j = 0; j < 3; ++j) {
+        const LD x = fmaxl(fmaxl((LD)lo[j] - q[j], (LD)q[j] - hi[j]), 0.0L);
+        d2 += x * x;
+      }
+      const double best = (double)sqrtl(d2);
+      const ClosestPointF c = closest_point(D3{q[0], q[1], q[2]}, closest_shrink(bump, ext));
+      const float d = closest_box(flo[0], fhi[0], flo[1], fhi[1], flo[2], fhi[2], c);
+      w += !(d <= closest_limit(best));
+      passed += d <= closest_limit(0.9 * best);
+      ++total;
+    }
+    if (w) std::printf("scale 1e%d: %ld of 20000 boxes at the best distance pruned\n", e, w);
+    wrong += w;
+  }
+  if (passed * 2 > total) {
+    std::printf("%ld of %ld farther boxes not pruned\n", passed, total);
+    ++wrong;
+  }
+  return wrong != 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -107,6 +149,7 @@ int main(int argc, char** argv)
   int rc = 1;
   if (argc == 2 && !std::strcmp(argv[1], "closest")) rc = closest_bound(-24, 24, false);
   if (argc == 2 && !std::strcmp(argv[1], "closest_thin")) rc = closest_bound(-24, 24, true);
+  if (argc == 2 && !std::strcmp(argv[1], "closest_boxes")) rc = closest_boxes();
   if (!rc) std::printf("ok\n");
   return rc;
 }

@@ -33,10 +33,11 @@ def check(ctx, v9, bump, pts, face=None):
     ctx.release_surface_tree(tree)
 
 
-@pytest.mark.parametrize("radius", [1e-11, 1e-9, 1e-5, 1.0, 1e5, 1e9, 1e10, 1e13])
+@pytest.mark.parametrize("radius", [1e-22, 1e-21, 1e-11, 1e-9, 1e-5, 1.0, 1e5, 1e9, 1e10, 1e13])
 @pytest.mark.parametrize("subdiv", [1, 3])
 def test_closest_scales(ctx, radius, subdiv):
-    """Products of four lengths leave FP32's range at both ends."""
+    """Products of four lengths leave FP32's range at both ends, squares its
+    normal range at the smallest radii."""
     v, t = G.icosphere(subdiv, radius)
     pts = P.ball_points(81, 0, 2000, 1.5 * radius)
     check(ctx, v[t].reshape(-1, 9), 1e-6 * radius, pts)

@@ -82,4 +82,39 @@ __host__ __device__ __forceinline__ bool closest_beyond(const D3& v0, const D3& 
   return m >= 0x1p-50f && m <= 0x1p60f && lb - 0x1p-17f * m > best2;
 }
 
+// A point against the BVH4's FP32 boxes.  The boxes were dilated by the
+// tree's bump; pm = p - s and pp = p + s with s just below the bump take that
+// back, so the distance to a box is that to its vertices' bounds.  pm is
+// rounded up and pp down, and the bump loses 2^-40 of the coordinates, more
+// than the rounding of a closest point: only relative roundings are left
+// (one difference, a square, two sums: 5 x 2^-24), which the factor on the
+// limit covers, and the absolute ones of squares below FP32's normal range,
+// which the addend covers.  A box whose distance exceeds the limit holds no triangle
+// at the best distance or below.
+struct ClosestPointF {
+  float mx, my, mz, px, py, pz;
+};
+__host__ __device__ __forceinline__ float closest_limit(double best)
+{
+  return f32_up(best * best) * (1.0f + 0x1p-21f) + 0x1p-126f;
+}
+__host__ __device__ __forceinline__ double closest_shrink(double bump, double max_abs)
+{
+  return bump - 0x1p-40 * (max_abs + bump);
+}
+__host__ __device__ __forceinline__ ClosestPointF closest_point(const D3& p, double s)
+{
+  return ClosestPointF{f32_up(p.x - s),     f32_up(p.y - s),     f32_up(p.z - s),
+                       f32_down_d(p.x + s), f32_down_d(p.y + s), f32_down_d(p.z + s)};
+}
+// squared distance to a box of the tree
+__host__ __device__ __forceinline__ float closest_box(float lx, float hx, float ly, float hy, float lz, float hz,
+                                                     const ClosestPointF& c)
+{
+  const float ex = fmaxf(fmaxf(lx - c.mx, c.px - hx), 0.0f);
+  const float ey = fmaxf(fmaxf(ly - c.my, c.py - hy), 0.0f);
+  const float ez = fmaxf(fmaxf(lz - c.mz, c.pz - hz), 0.0f);
+  return ex * ex + ey * ey + ez * ez;
+}
+
 }  // namespace xdgd

@@ -616,21 +616,6 @@ __device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* 
   }
 }
 
-// A point against the BVH4's FP32 boxes.  The boxes were dilated by the
-// tree's bump; pm = p - s and pp = p + s with s just below the bump take that
-// back, so the distance to a box is that to its vertices' bounds.  pm is
-// rounded up and pp down, and the bump loses 2^-40 of the coordinates, more
-// than the rounding of a closest point: only relative roundings are left
-// (one difference, a square, two sums: 5 x 2^-24), which the factor on the
-// limit covers.  A box whose distance exceeds the limit holds no triangle
-// at the best distance or below.
-struct ClosestPointF {
-  float mx, my, mz, px, py, pz;
-};
-__device__ __forceinline__ float closest_limit(double best)
-{
-  return f32_up(best * best) * (1.0f + 0x1p-21f);
-}
 // children within the limit, nearest first (others CHILD_EMPTY)
 __device__ __forceinline__ void node4_dist(const Node4F* nodes, int32_t node, const ClosestPointF& c, float lim,
                                            float* te, int32_t* ch)
@@ -646,10 +631,7 @@ __device__ __forceinline__ void node4_dist(const Node4F* nodes, int32_t node, co
   const int32_t cca[4] = {cc.x, cc.y, cc.z, cc.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float ex = fmaxf(fmaxf(lxa[i] - c.mx, c.px - hxa[i]), 0.0f);
-    const float ey = fmaxf(fmaxf(lya[i] - c.my, c.py - hya[i]), 0.0f);
-    const float ez = fmaxf(fmaxf(lza[i] - c.mz, c.pz - hza[i]), 0.0f);
-    const float d = ex * ex + ey * ey + ez * ez;
+    const float d = closest_box(lxa[i], hxa[i], lya[i], hya[i], lza[i], hza[i], c);
     const bool in = d <= lim && cca[i] != CHILD_EMPTY;
     te[i] = in ? d : INFINITY;
     ch[i] = in ? cca[i] : CHILD_EMPTY;
@@ -741,7 +723,7 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int 
   const SurfTreeDev T = a.table[a.tree];
   double ext = 0.0;
   for (int k = 0; k < 3; ++k) ext = fmax(ext, fmax(fabs((double)T.box_lo[k]), fabs((double)T.box_hi[k])));
-  const double shrink = T.bump - 0x1p-40 * (ext + T.bump);
+  const double shrink = closest_shrink(T.bump, ext);
   const double limit = (double)T.o_limit;
   WaveStride w(a.n, lanes_first);
   while (!w.dry) {
@@ -762,8 +744,7 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int 
       L.px[lane] = p.x;
       L.py[lane] = p.y;
       L.pz[lane] = p.z;
-      L.c[lane] = ClosestPointF{f32_up(p.x - shrink),     f32_up(p.y - shrink),     f32_up(p.z - shrink),
-                                f32_down_d(p.x + shrink), f32_down_d(p.y + shrink), f32_down_d(p.z + shrink)};
+      L.c[lane] = closest_point(p, shrink);
       L.best[lane] = (unsigned long long)__double_as_longlong(best);
       L.face[lane] = bface;
       L.lim[lane] = INFINITY;
