@@ -142,6 +142,66 @@ int closest_boxes()
   return wrong != 0;
 }
 
+// the FP64 test of a ray against a box that carries its slack
+bool slab64(const double* lo, const double* hi, const double* o, const double* d)
+{
+  double a = 0.0, b = INFTY;
+  for (int k = 0; k < 3; ++k) {
+    if (d[k] == 0.0) {
+      if (o[k] < lo[k] || o[k] > hi[k]) return false;
+      continue;
+    }
+    const double inv = 1.0 / d[k], t0 = (lo[k] - o[k]) * inv, t1 = (hi[k] - o[k]) * inv;
+    a = std::fmax(a, std::fmin(t0, t1));
+    b = std::fmin(b, std::fmax(t0, t1));
+  }
+  return a <= b;
+}
+
+// The start stage's boxes: a box that the FP64 test reaches is reached
+// (coordinates 10^lo to 10^hi, near-axis and axis-parallel directions, aimed
+// at corners and edges, where a miss is nearest), and a slot without hits
+// never is.
+int start_boxes(double lo_exp, double hi_exp)
+{
+  long dropped = 0, reached = 0, none = 0;
+  const int n = 400000;
+  for (int i = 0; i < n; ++i) {
+    const double scale = std::pow(10.0, lo_exp + (hi_exp - lo_exp) * uni());
+    const double half = scale * std::pow(10.0, -4.0 * uni()), bump = 1e-3 * uni();
+    float blo[3], bhi[3], box[6], empty[6];
+    double slo[3], shi[3], o[3], d[3], wlo[3], whi[3], len = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      slo[k] = -scale * uni();
+      shi[k] = scale * uni();
+      o[k] = slo[k] + (shi[k] - slo[k]) * uni();
+      const double mid = scale * (4.0 * uni() - 2.0), h = half * uni();
+      blo[k] = f32_down_d(mid - h);
+      bhi[k] = f32_up(mid + h);
+      const double slack = 2.0 * bump + 0x1p-30 * (std::fabs((double)blo[k]) + std::fabs((double)bhi[k]) + 1.0);
+      wlo[k] = blo[k] - slack;
+      whi[k] = bhi[k] + slack;
+      d[k] = i % 5 == 0 ? nrm() : (uni() < 0.5 ? wlo[k] : whi[k]) - o[k];
+    }
+    if (i % 7 == 0) d[0] = i % 2 ? 0.0 : -0.0;
+    for (int k = 0; k < 3; ++k) len += d[k] / scale * (d[k] / scale);
+    for (int k = 0; k < 3; ++k) d[k] /= scale * std::sqrt(len);
+    if (i % 7 == 1) d[1] *= 1e-33;
+    start_box(blo, bhi, bump, slo, shi, box);
+    start_box_none(empty);
+    const float3 fo = make_float3((float)o[0], (float)o[1], (float)o[2]);
+    const float3 inv = make_float3(safe_inv_f((float)d[0]), safe_inv_f((float)d[1]), safe_inv_f((float)d[2]));
+    const bool ref = slab64(wlo, whi, o, d);
+    reached += ref;
+    dropped += ref && !start_box_hit(box, fo, inv);
+    none += start_box_hit(empty, fo, inv);
+  }
+  if (dropped) std::printf("%ld of %ld reached boxes dropped\n", dropped, reached);
+  if (none) std::printf("%ld of %d rays reach a slot without hits\n", none, n);
+  if (reached < n / 10) std::printf("only %ld boxes reached\n", reached);
+  return dropped || none || reached < n / 10;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -150,6 +210,7 @@ int main(int argc, char** argv)
   if (argc == 2 && !std::strcmp(argv[1], "closest")) rc = closest_bound(-24, 24, false);
   if (argc == 2 && !std::strcmp(argv[1], "closest_thin")) rc = closest_bound(-24, 24, true);
   if (argc == 2 && !std::strcmp(argv[1], "closest_boxes")) rc = closest_boxes();
+  if (argc == 2 && !std::strcmp(argv[1], "start_boxes")) rc = start_boxes(-3.0, 6.0);
   if (!rc) std::printf("ok\n");
   return rc;
 }

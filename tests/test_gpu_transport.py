@@ -339,6 +339,33 @@ def test_transport_over_1024_volumes(ctx, start_form):
             ctx.release_surface_tree(t)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+def test_transport_slots_without_hits(ctx, lattice, prec, start_form):
+    """The implicit complement first in the volume list, with a tree around
+    the whole lattice, and a volume with an empty tree: no start form takes
+    either as a start volume, whether the items fit their buffer or not."""
+    m, vols, trees, otrees = lattice
+    empty = (np.zeros((0, 9)), np.zeros(0, np.int32), np.zeros(0, np.int32), np.zeros(0, np.uint8))
+    none = ctx.build_surface_tree(np.zeros((0, 3)), np.zeros((0, 3), np.int32), *empty[1:], 1e-3)
+    ids = [m.ipc] + vols[:5] + [max(m.volumes) + 1] + vols[5:]
+    box = vols.index(max(vols))  # the region around the spheres contains their points too
+    gt = [trees[box]] + trees[:5] + [none] + trees[5:]
+    ot = [otrees[box]] + otrees[:5] + [O.Tree(*empty, 1e-3)] + otrees[5:]
+    h = ctx.transport_create(ids, gt, m.ipc, m.senses, SEED, STREAM, [0.0] * 3, [6.0] * 3, 2.0, 0.3, 10000)
+    try:
+        n = 4000
+        r = O.transport(m, ot, ids, SEED, STREAM, [0.0] * 3, [6.0] * 3, 2.0, 0.3, 10000, 0, n)
+        assert (r["tally_fx"][[0, 6]] == 0).all() and (r["status"] == 1).sum() > 1000
+        for staged, items, events in [(0, 8, 1), (1, 8, 0), (2, 8, 1), (2, 8, 0), (2, 1, 1)]:
+            ctx.set_option("transport_start", staged)
+            ctx.set_option("transport_items", items)
+            ctx.set_option("transport_events", events)
+            _check(ctx.transport_run(h, 0, n, len(ids), precision=prec), r)
+    finally:
+        ctx.transport_destroy(h)
+        ctx.release_surface_tree(none)
+
+
 def test_transport_prefilter_far_from_origin(ctx, start_form):
     """A sphere 3e5 from the origin, its trees built with a 1e-3 bump (the
     C-ABI takes any bump), and every start sampled 0.005 inside the

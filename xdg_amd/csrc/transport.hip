@@ -21,6 +21,7 @@
 
 #include <algorithm>
 
+#include "fp32_bounds.h"
 #include "internal.h"
 #include "surface_traverse.h"
 
@@ -82,46 +83,18 @@ __device__ __forceinline__ bool may_hit_tree(const SurfTreeDev& T, const D3& o, 
   return a <= b;
 }
 
-// may_hit_tree's dilated box of every volume slot, written at each launch
-// from the live tree table (a refit moves the boxes), for an FP32 slab test
-// of rays from the source box: outward-rounded, with 2^-19 of the largest
-// coordinates on either side as further slack.  The test's rounding moves a
-// plane by at most 5 x 2^-24 of |plane| + |origin|, so its boxes never miss
-// one that may_hit_tree's would reach.  A slot that can hold no hit (the
-// implicit complement, an unknown or empty tree) gets an inverted box.
+// The prefilter box (start_box) of every volume slot, written at each launch
+// from the live tree table (a refit moves the boxes).
 __global__ void k_transport_prefilter(TransportDev P, float* box)
 {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= P.nvol) return;
   const int32_t t = P.vol_tree[v];
-  bool ok = P.vol_id[v] != P.ipc && t >= 1 && t <= P.ntrees;
-  const SurfTreeDev* T = ok ? &P.table[t] : nullptr;
-  ok = ok && T->n_prims > 0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    float lo = INFINITY, hi = -INFINITY;
-    if (ok) {
-      const double ext = fabs((double)T->box_lo[k]) + fabs((double)T->box_hi[k]) + 1.0;
-      const double slack = 2.0 * T->bump + 0x1p-30 * ext + 0x1p-19 * (ext + fabs(P.lo[k]) + fabs(P.hi[k]));
-      lo = f32_down_d((double)T->box_lo[k] - slack);
-      hi = f32_up((double)T->box_hi[k] + slack);
-    }
-    box[6 * v + k] = lo;
-    box[6 * v + 3 + k] = hi;
-  }
-}
-
-// Slab test of a prefilter box (inv is finite, so no product is NaN).  FP64
-// and a branch per axis bound the counting pass by VALU issue: 2^20 histories
-// x 513 boxes 1.17 -> 0.40 ms.
-__device__ __forceinline__ bool may_hit_box(const float* b, const float3& o, const float3& inv)
-{
-  const float x0 = (b[0] - o.x) * inv.x, x1 = (b[3] - o.x) * inv.x;
-  const float y0 = (b[1] - o.y) * inv.y, y1 = (b[4] - o.y) * inv.y;
-  const float z0 = (b[2] - o.z) * inv.z, z1 = (b[5] - o.z) * inv.z;
-  const float a = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
-  const float e = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1));
-  return a <= e;
+  const bool known = P.vol_id[v] != P.ipc && t >= 1 && t <= P.ntrees;
+  if (known && P.table[t].n_prims > 0)
+    start_box(P.table[t].box_lo, P.table[t].box_hi, P.table[t].bump, P.lo, P.hi, box + 6 * v);
+  else
+    start_box_none(box + 6 * v);
 }
 
 __device__ __forceinline__ int wave_min_i(int x)
@@ -306,7 +279,7 @@ __device__ __forceinline__ uint64_t cand_mask(const TransportDev& P, const Trans
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (open)
     for (int q = 0; q < cn; ++q)
-      if (may_hit_box(wbox + 6 * q, o, inv)) m |= 1ull << q;
+      if (start_box_hit(wbox + 6 * q, o, inv)) m |= 1ull << q;
   if (keep && open) G.masks[(int64_t)(v0 >> 6) * G.cap + j] = m;
   __builtin_amdgcn_wave_barrier();
   return m;
