@@ -189,7 +189,7 @@ int start_boxes(double lo_exp, double hi_exp)
     if (i % 7 == 1) d[1] *= 1e-33;
     start_box(blo, bhi, bump, slo, shi, box);
     start_box_none(empty);
-    const float3 fo = make_float3((float)o[0], (float)o[1], (float)o[2]);
+    const float3 fo = make_float3(start_coord(o[0]), start_coord(o[1]), start_coord(o[2]));
     const float3 inv = make_float3(safe_inv_f((float)d[0]), safe_inv_f((float)d[1]), safe_inv_f((float)d[2]));
     const bool ref = slab64(wlo, whi, o, d);
     reached += ref;
@@ -211,6 +211,7 @@ int main(int argc, char** argv)
   if (argc == 2 && !std::strcmp(argv[1], "closest_thin")) rc = closest_bound(-24, 24, true);
   if (argc == 2 && !std::strcmp(argv[1], "closest_boxes")) rc = closest_boxes();
   if (argc == 2 && !std::strcmp(argv[1], "start_boxes")) rc = start_boxes(-3.0, 6.0);
+  if (argc == 2 && !std::strcmp(argv[1], "start_boxes_huge")) rc = start_boxes(6.0, 60.0);
   if (!rc) std::printf("ok\n");
   return rc;
 }

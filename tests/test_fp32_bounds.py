@@ -18,7 +18,7 @@ def exe(tmp_path_factory):
     return str(out)
 
 
-@pytest.mark.parametrize("check", ["closest", "closest_thin", "closest_boxes", "start_boxes"])
+@pytest.mark.parametrize("check", ["closest", "closest_thin", "closest_boxes", "start_boxes", "start_boxes_huge"])
 def test_bound(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -123,17 +123,30 @@ __host__ __device__ __forceinline__ float closest_box(float lx, float hx, float 
 // [src_lo, src_hi]: outward-rounded, with 2^-19 of the largest coordinates on
 // either side as further slack.  The test's rounding moves a plane by at most
 // 5 x 2^-24 of |plane| + |origin|, so its boxes never miss one that the FP64
-// test would reach.
+// test would reach.  Coordinates near FP32's range or beyond it, whose
+// differences it does not hold, give a box that every ray reaches.
 __host__ __device__ __forceinline__ void start_box(const float* lo, const float* hi, double bump, const double* src_lo,
                                                   const double* src_hi, float* box)
 {
+  double most = 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const double ext = fabs((double)lo[k]) + fabs((double)hi[k]) + 1.0;
-    const double slack = 2.0 * bump + 0x1p-30 * ext + 0x1p-19 * (ext + fabs(src_lo[k]) + fabs(src_hi[k]));
+    const double ext = fabs((double)lo[k]) + fabs((double)hi[k]) + 1.0 + fabs(src_lo[k]) + fabs(src_hi[k]);
+    const double slack = 2.0 * bump + (0x1p-30 + 0x1p-19) * ext;
     box[k] = f32_down_d((double)lo[k] - slack);
     box[3 + k] = f32_up((double)hi[k] + slack);
+    most = fmax(most, ext + slack);
   }
+  if (!(most <= 0x1p120))
+    for (int k = 0; k < 3; ++k) {
+      box[k] = -INFINITY;
+      box[3 + k] = INFINITY;
+    }
+}
+// a ray's origin for the slab test, finite
+__host__ __device__ __forceinline__ float start_coord(double x)
+{
+  return fminf(fmaxf((float)x, -0x1.fffffep127f), 0x1.fffffep127f);
 }
 // The box of a slot that can hold no hit (the implicit complement, an unknown
 // or empty tree): inverted.  The slab test orders the planes of an axis
@@ -146,9 +159,9 @@ __host__ __device__ __forceinline__ void start_box_none(float* box)
     box[3 + k] = -INFINITY;
   }
 }
-// Slab test of such a box (inv is finite, so no product is NaN).  FP64 and a
-// branch per axis bound the counting pass by VALU issue: 2^20 histories x 513
-// boxes 1.17 -> 0.40 ms.
+// Slab test of such a box (o and inv are finite, so no product is NaN).  FP64
+// and a branch per axis bound the counting pass by VALU issue: 2^20 histories
+// x 513 boxes 1.17 -> 0.40 ms.
 __host__ __device__ __forceinline__ bool start_box_hit(const float* b, const float3& o, const float3& inv)
 {
   const float x0 = (b[0] - o.x) * inv.x, x1 = (b[3] - o.x) * inv.x;

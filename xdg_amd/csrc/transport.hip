@@ -344,7 +344,7 @@ __global__ __launch_bounds__(CAND_BLOCK) void k_transport_cand(TransportDev P, T
     load_start(G, i, r, u);
     open = true;
   }
-  const float3 o = make_float3((float)r.x, (float)r.y, (float)r.z);
+  const float3 o = make_float3(start_coord(r.x), start_coord(r.y), start_coord(r.z));
   const float3 inv = make_float3(safe_inv_f((float)u.x), safe_inv_f((float)u.y), safe_inv_f((float)u.z));
   const bool any = __ballot(open) != 0;  // wave-uniform
   const bool keep = G.mask_words > 0;
