@@ -1045,7 +1045,18 @@ struct C4Item {
   int32_t bnode;  // binary node this BVH4 node is built from
   int32_t slot;   // BVH4 node index
   int32_t above;  // stack entries pushed above it on its path
+  int32_t level;  // bnode's level in the binary tree (root 1)
 };
+
+// Children a BVH4 node may have so that the stack stays within limit
+// entries: below it at least one child per remaining binary level is pushed
+// (a tree opened to binary nodes only needs its depth).  Never below 2 while
+// the binary depth is at most limit.
+__device__ __forceinline__ int c4_most(const C4Item& it, int32_t depth, int32_t limit)
+{
+  const int32_t k = limit - it.above - (depth - it.level) + 1;
+  return k < 2 ? 2 : (k < 4 ? k : 4);
+}
 
 __device__ __forceinline__ double half_area_d(const double* b)
 {
@@ -1058,16 +1069,18 @@ __device__ __forceinline__ const double* src_box(const NodeD* nd, int32_t src)
   return (src & 1) ? nd[src >> 1].b1 : nd[src >> 1].b0;
 }
 
-// children of the BVH4 node over binary node b: codes and box sources
-__device__ __forceinline__ int c4_children(const NodeD* __restrict__ nd, int64_t n_nodes, int32_t b, int32_t* code,
-                                           int32_t* src, bool* bad)
+// children of the BVH4 node over binary node b (at most `most`): codes, box
+// sources and binary levels below b's
+__device__ __forceinline__ int c4_children(const NodeD* __restrict__ nd, int64_t n_nodes, int32_t b, int most,
+                                           int32_t* code, int32_t* src, int32_t* below, bool* bad)
 {
+  below[0] = below[1] = 1;
   code[0] = nd[b].c0;
   src[0] = 2 * b;
   code[1] = nd[b].c1;
   src[1] = 2 * b + 1;
   int nc = 2;
-  while (nc < 4) {
+  while (nc < most) {
     int best = -1;
     double area = -1.0;
     for (int j = 0; j < nc; ++j)
@@ -1088,19 +1101,20 @@ __device__ __forceinline__ int c4_children(const NodeD* __restrict__ nd, int64_t
     src[best] = 2 * x;
     code[nc] = nd[x].c1;
     src[nc] = 2 * x + 1;
+    below[nc] = ++below[best];
     ++nc;
   }
   return nc;
 }
 
 __global__ void k_c4_count(const NodeD* __restrict__ nd, int64_t n_nodes, const C4Item* __restrict__ items,
-                           unsigned int nitems, uint32_t* cnt, unsigned int* err)
+                           unsigned int nitems, int32_t depth, int32_t limit, uint32_t* cnt, unsigned int* err)
 {
   const unsigned int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nitems) return;
-  int32_t code[4], src[4];
+  int32_t code[4], src[4], below[4];
   bool bad = items[i].bnode < 0 || items[i].bnode >= n_nodes;
-  int nc = bad ? 0 : c4_children(nd, n_nodes, items[i].bnode, code, src, &bad);
+  int nc = bad ? 0 : c4_children(nd, n_nodes, items[i].bnode, c4_most(items[i], depth, limit), code, src, below, &bad);
   uint32_t k = 0;
   for (int j = 0; j < nc; ++j) k += code[j] >= 0 ? 1u : 0u;
   if (bad) {
@@ -1112,7 +1126,8 @@ __global__ void k_c4_count(const NodeD* __restrict__ nd, int64_t n_nodes, const 
 
 __global__ void k_c4_emit(const NodeD* __restrict__ nd, const NodeF* __restrict__ nf, int64_t n_nodes, int64_t n,
                           const C4Item* __restrict__ items, unsigned int nitems, const uint32_t* __restrict__ offs,
-                          int32_t next_base, int64_t cap, Node4D* o4d, Node4F* o4f, int32_t* src4, C4Item* next,
+                          int32_t depth, int32_t limit, int32_t next_base, int64_t cap, Node4D* o4d, Node4F* o4f,
+                          int32_t* src4, C4Item* next,
                           unsigned int* seen, int* max_stack, unsigned int* err)
 {
   const unsigned int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1122,9 +1137,9 @@ __global__ void k_c4_emit(const NodeD* __restrict__ nd, const NodeF* __restrict_
     atomicOr(err, 1u);
     return;
   }
-  int32_t code[4], src[4];
+  int32_t code[4], src[4], below[4];
   bool bad = it.bnode < 0 || it.bnode >= n_nodes;
-  const int nc = bad ? 0 : c4_children(nd, n_nodes, it.bnode, code, src, &bad);
+  const int nc = bad ? 0 : c4_children(nd, n_nodes, it.bnode, c4_most(it, depth, limit), code, src, below, &bad);
   if (bad) {
     atomicOr(err, 1u);
     return;
@@ -1154,7 +1169,7 @@ __global__ void k_c4_emit(const NodeD* __restrict__ nd, const NodeF* __restrict_
       f4.hiz[j] = bf[5];
       if (code[j] >= 0) {
         const int32_t slot = next_base + (int32_t)(offs[i] + rank);
-        next[offs[i] + rank] = C4Item{code[j], slot, above};
+        next[offs[i] + rank] = C4Item{code[j], slot, above, it.level + below[j]};
         ++rank;
         d4.child[j] = f4.child[j] = slot;
       } else {
@@ -1217,7 +1232,7 @@ __global__ void k_copy_bytes16(const uint4* __restrict__ src, uint4* dst, int64_
 }  // namespace
 
 void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<DevBuf>& owned, Bvh4Out& out,
-                   bool keep_sources, bool fp64_nodes)
+                   bool keep_sources, bool fp64_nodes, int32_t max_stack)
 {
   if (bin.root < 0 || bin.n_nodes == 0) {  // a single leaf: no nodes
     out.root = bin.root;
@@ -1241,21 +1256,21 @@ void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<Dev
     auto* misc = (unsigned int*)dev_alloc(sizeof(unsigned int) * 4, tmp);  // total, err, max_stack
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n)), dim3(BLK), 0, s, seen, n, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, misc, 4, 0u);
-    const C4Item root{bin.root, 0, 0};
+    const C4Item root{bin.root, 0, 0, 1};
     XDG_HIP_CHECK(hipMemcpyAsync(lv0, &root, sizeof root, hipMemcpyHostToDevice, s));
     unsigned int nin = 1;
     int64_t slots = 1;
     for (int level = 0; nin > 0; ++level) {
       if (level > 64) throw HipError{"bvh4: deeper than 64 levels"};
-      hipLaunchKernelGGL(k_c4_count, dim3(grid_for(nin)), dim3(BLK), 0, s, bin.nodes_d, bin.n_nodes, lv0, nin, cnt,
-                         misc + 1);
+      hipLaunchKernelGGL(k_c4_count, dim3(grid_for(nin)), dim3(BLK), 0, s, bin.nodes_d, bin.n_nodes, lv0, nin,
+                         bin.depth, max_stack, cnt, misc + 1);
       hipLaunchKernelGGL(k_scan_excl, dim3(1), dim3(1024), 0, s, cnt, (int64_t)nin, misc);
       unsigned int total = 0;
       XDG_HIP_CHECK(hipMemcpyAsync(&total, misc, sizeof total, hipMemcpyDeviceToHost, s));
       XDG_HIP_CHECK(hipStreamSynchronize(s));
       if (slots + (int64_t)total > cap) throw HipError{"bvh4: more nodes than the binary tree has"};
       hipLaunchKernelGGL(k_c4_emit, dim3(grid_for(nin)), dim3(BLK), 0, s, bin.nodes_d, bin.nodes_f, bin.n_nodes, n,
-                         lv0, nin, cnt, (int32_t)slots, cap, t4d, t4f, tsrc, lv1, seen, (int*)(misc + 2), misc + 1);
+                         lv0, nin, cnt, bin.depth, max_stack, (int32_t)slots, cap, t4d, t4f, tsrc, lv1, seen, (int*)(misc + 2), misc + 1);
       slots += total;
       nin = total;
       std::swap(lv0, lv1);

@@ -334,11 +334,13 @@ int surf_need(xdg_hip_ctx* c, const SurfTreeHost* t)
   return t ? t->dev.depth : c->max_surf_depth;
 }
 
+constexpr int MAX_STACK = 64;
+
 LaunchCfg cfg_for(xdg_hip_ctx* c, int depth)
 {
   LaunchCfg k = c->cfg;
   k.stack = std::max(k.stack, std::max(depth, 1));
-  if (k.stack > 64) throw InvalidArg{"tree deeper than the 64-entry traversal stack"};
+  if (k.stack > MAX_STACK) throw InvalidArg{"tree deeper than the 64-entry traversal stack"};
   // keep the LDS stack within 64 KiB per workgroup
   while ((size_t)(k.stack + GUARDED_STACK_EXTRA) * k.block * 4 > 65536 && k.block > 64) k.block /= 2;
   return k;
@@ -850,7 +852,9 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
       XDG_HIP_CHECK(hipGetLastError());
       XDG_HIP_CHECK(hipStreamSynchronize(s));
       Bvh4Out b4;
-      bvh4_collapse(lb, n_tets, s, t.bufs, b4, false, false);
+      // there is no other tree to query: its stack bound stays within what
+      // queries accept, as the binary tree's depth does
+      bvh4_collapse(lb, n_tets, s, t.bufs, b4, false, false, MAX_STACK);
       // queries read the FP32 BVH4 alone
       for (void* p : {(void*)lb.nodes_d, (void*)lb.nodes_f}) dev_free_one(t.bufs, p);
       t.dev.nodes4_f = b4.nodes_f;
@@ -1312,7 +1316,7 @@ int xdg_hip_closest(xdg_hip_ctx* c, int32_t tree, int64_t n, const double* pts, 
     if (n == 0) return XDG_HIP_OK;
     require(pts && dist_out && face_out, "null array");
     ClosestArgs a{c->d_surf, (int32_t)c->surf.size(), tree, n, pts, dist_out, face_out};
-    launch_closest(a, cfg_for(c, std::max(t.dev.depth, t.dev.stack4)), pick(c, stream));
+    launch_closest(a, cfg_for(c, t.dev.depth), t.dev.stack4, pick(c, stream));
     XDG_HIP_CHECK(hipGetLastError());
     return XDG_HIP_OK;
   });

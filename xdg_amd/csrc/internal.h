@@ -86,7 +86,9 @@ void lbvh_build(const double* box6, int64_t n, int leaf_max, hipStream_t s, std:
 void lbvh_refit(const double* box6, int64_t n, LbvhOut& out, hipStream_t s);
 
 // 4-wide tree over the same leaves, collapsed from a binary LBVH on the
-// device, level by level.
+// device, level by level.  Each node opens children until it has four, which
+// pushes up to three entries for two binary levels; where the stack would
+// exceed max_stack (at least the binary depth) a node keeps fewer.
 struct Bvh4Out {
   xdgd::Node4D* nodes_d = nullptr;
   xdgd::Node4F* nodes_f = nullptr;
@@ -96,7 +98,7 @@ struct Bvh4Out {
   int32_t* src = nullptr;  // 4 per node: binary (node << 1 | side) each child box comes from, -1 empty
 };
 void bvh4_collapse(const LbvhOut& bin, int64_t n, hipStream_t s, std::vector<DevBuf>& owned, Bvh4Out& out,
-                   bool keep_sources = false, bool fp64_nodes = true);
+                   bool keep_sources = false, bool fp64_nodes = true, int32_t max_stack = 1 << 20);
 // Child boxes of the BVH4 copied again from the (refitted) binary nodes.
 void bvh4_refit(const LbvhOut& bin, const Bvh4Out& b4, hipStream_t s);
 
@@ -260,7 +262,8 @@ struct ClosestArgs {
   double* dist;
   int32_t* face;
 };
-void launch_closest(const ClosestArgs& a, const LaunchCfg& c, hipStream_t s);
+// stack4: the tree's BVH4 stack bound (c.stack holds the binary depth)
+void launch_closest(const ClosestArgs& a, const LaunchCfg& c, int stack4, hipStream_t s);
 
 // ---- batched particle random walk (transport.hip) -------------------------
 // Device-resident problem (arrays owned by the context's transport handle).

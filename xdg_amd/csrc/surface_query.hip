@@ -647,6 +647,8 @@ __device__ __forceinline__ void node4_dist(const Node4F* nodes, int32_t node, co
 // A queue entry is a child code and a tag: the point's lane, and the upper
 // half of the entry's FP32 box distance (a lower bound).
 constexpr int CLOSEST_NODES = 1536;  // node queue
+constexpr int CLOSEST_STACK_MAX = 192;  // stack bound of any BVH4: three entries for each of 64 levels
+static_assert(CLOSEST_NODES >= 64 + 3 * 64 + CLOSEST_STACK_MAX, "a wave's points and one full step fit the queue");
 constexpr int CLOSEST_LEAVES = 320;  // leaf queue: below 64, plus one step's 4 x 64
 struct ClosestLds {
   double px[64], py[64], pz[64];
@@ -709,13 +711,14 @@ __device__ __forceinline__ void closest_push(ClosestLds& L, int owner, const flo
 //
 // Steps take nodes while fewer than 64 leaves wait, else leaves.  While the
 // node queue has no room for a full step's pushes (3 x 64 net) above
-// `reserve` entries, nodes are taken one at a time: depth first, at most
-// the tree's stack bound more entries, so it cannot overflow.
+// `reserve` entries (the BVH4's stack bound), nodes are taken one at a time:
+// depth first, at most that many more entries, so it cannot overflow.  cap
+// is the binary tree's depth, for the FP64 descents.
 // 100 003 points in a ball around a sphere of 20 480 triangles: 7.4 -> 0.35 ms
 // (a descent per lane on these boxes, the last 16 points of a wave finished
 // by all its lanes: 0.73 ms).  Bound by the latency of the steps, two waves
 // per SIMD (19 KB of LDS each).
-__global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int lanes_first)
+__global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int cap, int reserve, int lanes_first)
 {
   extern __shared__ __align__(16) unsigned char smem[];
   ClosestLds& L = *(ClosestLds*)smem;
@@ -739,7 +742,7 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int 
         if (fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z)) <= limit)
           queued = true;
         else
-          closest_fp64(T, p, L.node + lane, 64, reserve, best, bface);
+          closest_fp64(T, p, L.node + lane, 64, cap, best, bface);
       }
       L.px[lane] = p.x;
       L.py[lane] = p.y;
@@ -1034,7 +1037,7 @@ void launch_occluded(const OccludedArgs& a, bool mixed, const LaunchCfg& c, hipS
   XDG_DISPATCH2(k_occluded, mixed, c.wide, grid1(a.n, c.block), dim3(c.block), lds_bytes(c), s, a, c.stack);
 }
 
-void launch_closest(const ClosestArgs& a, const LaunchCfg& c, hipStream_t s)
+void launch_closest(const ClosestArgs& a, const LaunchCfg& c, int stack4, hipStream_t s)
 {
   if (a.n <= 0) return;
   const size_t sh = offsetof(ClosestLds, node) + sizeof(int32_t) * (size_t)std::max(CLOSEST_NODES, 64 * c.stack);
@@ -1043,7 +1046,7 @@ void launch_closest(const ClosestArgs& a, const LaunchCfg& c, hipStream_t s)
   const int64_t waves = resident_grid(k_closest, 64, sh);
   const int lanes_first = (int)std::min<int64_t>(64, (a.n + waves - 1) / waves);
   const unsigned grid = (unsigned)std::min<int64_t>(waves, (a.n + lanes_first - 1) / lanes_first);
-  hipLaunchKernelGGL(k_closest, dim3(grid), dim3(64), sh, s, a, c.stack, lanes_first);
+  hipLaunchKernelGGL(k_closest, dim3(grid), dim3(64), sh, s, a, c.stack, stack4, lanes_first);
 }
 
 // ---- primitive evaluation (parity checks of the device geometry kernels) --
