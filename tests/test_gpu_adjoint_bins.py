@@ -52,3 +52,39 @@ def test_binned_adjoint(ctx, ntri, n, crowd):
     assert np.array_equal(bits(host(go)), bits(oo)) and np.array_equal(bits(host(gd)), bits(od))
     # at most n terms of the largest vertex sum's size, each rounded a few times
     assert np.allclose(host(gv), ov, rtol=1e-12, atol=1e-12 * np.abs(ov).max())
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e300, -1e305])
+def test_binned_adjoint_extreme_weights(ctx, value):
+    """Infinite, NaN and huge dL/dt on a few rays: every vertex component is
+    infinite, NaN or finite as the sum of single rays' terms is."""
+    m = G.perturbed_sphere(3, 10.0, 0.05)
+    n = 70000
+    rng = np.random.default_rng(89)
+    face = rng.integers(0, len(m.tris), n).astype(np.int32)
+    v = m.verts[m.tris[face]]
+    b = rng.random((n, 2)) * 0.5
+    hit = v[:, 0] + b[:, :1] * (v[:, 1] - v[:, 0]) + b[:, 1:] * (v[:, 2] - v[:, 0])
+    org = P.ball_points(9, 0, n, 9.0)
+    t = np.linalg.norm(hit - org, axis=1)
+    dirs = (hit - org) / t[:, None]
+    w = rng.standard_normal(n)
+    w[::9001] = value
+    gv = torch.zeros((m.verts.shape[0], 3), dtype=torch.float64, device="cuda")
+    go = torch.empty((n, 3), dtype=torch.float64, device="cuda")
+    gd = torch.empty_like(go)
+    ctx.ray_distance_adjoint(dev(torch, org), dev(torch, dirs), dev(torch, t), dev(torch, face), dev(torch, w),
+                             dev(torch, m.verts), dev(torch, m.tris), gv, go, gd)
+    ov, oo, od = O.adjoint(m.verts, m.tris, org, dirs, t, face, w)
+    gv = host(gv)
+    assert np.array_equal(host(go), oo, equal_nan=True) and np.array_equal(host(gd), od, equal_nan=True)
+    if not np.isfinite(value):
+        assert (~np.isfinite(ov)).sum() > 20
+    assert np.array_equal(np.isnan(gv), np.isnan(ov)) and np.array_equal(np.isinf(gv), np.isinf(ov))
+    inf, fin = np.isinf(ov), np.isfinite(ov)
+    assert np.array_equal(gv[inf], ov[inf])
+    big = np.zeros(len(gv), bool)
+    big[m.tris[face[::9001]]] = True
+    for part in (fin & big[:, None], fin & ~big[:, None]):
+        scale = np.abs(ov[part]).max(initial=0.0)
+        assert np.allclose(gv[part], ov[part], rtol=1e-12, atol=1e-12 * scale)

@@ -172,6 +172,10 @@ constexpr int ADJ_FACES = 256;      // faces per bucket: 8 KB of sums in LDS
 constexpr int ADJ_RAY_BLOCK = 512;  // k_adj_rays: rays per workgroup = ADJ_RAY_BLOCK * ADJ_RAYS
 constexpr int ADJ_RAYS = 4;
 constexpr int ADJ_CHUNK = 16384;    // k_adj_faces: rays per workgroup at most
+// A ray with a larger (or NaN) w or w q adds its own vertex terms: an
+// infinite sum of w q would make them NaN where they are infinite one by one,
+// and sums of 2^31 smaller ones, times edges of up to 2^190, do not overflow.
+constexpr double ADJ_SUM_MAX = 0x1p800;
 
 __device__ __forceinline__ bool adj_hit(const AdjointArgs& a, int64_t i, int32_t& f)
 {
@@ -267,8 +271,15 @@ __global__ __launch_bounds__(ADJ_RAY_BLOCK) void k_adj_rays(AdjointArgs a, Adjoi
     if (i < a.n) {
       AdjTerms A;
       if (adjoint_ray(a, i, A)) {
-        w[k] = A.w;
-        wq[k] = A.wq;
+        if (fabs(A.w) <= ADJ_SUM_MAX && fabs(A.wq.x) <= ADJ_SUM_MAX && fabs(A.wq.y) <= ADJ_SUM_MAX &&
+            fabs(A.wq.z) <= ADJ_SUM_MAX) {
+          w[k] = A.w;
+          wq[k] = A.wq;
+        } else {
+          add_vertex(a.dldv, A.i1, A.g1);
+          add_vertex(a.dldv, A.i2, A.g2);
+          add_vertex(a.dldv, A.i0, A.g0);
+        }
       }
       int32_t f;
       if (adj_hit(a, i, f)) {  // as counted: a hit without terms adds zeros
@@ -331,11 +342,7 @@ __global__ __launch_bounds__(256) void k_adj_faces(AdjointArgs a, AdjointBins b)
     add_exact(&sum[3][f], &err[3][f], e.z);
   }
   __syncthreads();
-  // an overflowed or NaN sum stays what it is (its error terms are NaN)
-  auto total = [&](int k) {
-    const double s = sum[k][threadIdx.x], c = s + err[k][threadIdx.x];
-    return fabs(s) < INFTY ? c : s;
-  };
+  auto total = [&](int k) { return sum[k][threadIdx.x] + err[k][threadIdx.x]; };
   const int64_t f = (int64_t)lo * ADJ_FACES + threadIdx.x;
   const double w = total(0);
   const D3 q = d3(total(1), total(2), total(3));
