@@ -482,8 +482,12 @@ int xdg_hip_transport_autotune(xdg_hip_ctx* ctx, int32_t handle, uint64_t first,
  * dldo[3 n] = dldt dt/do, dldd[3 n] = dldt dt/dd (zero for misses), with
  * t = n.(v0 - o)/(n.d), n = (v1 - v0) x (v2 - v0).  All arrays device,
  * dldv/dldo/dldd nullable.  Asynchronous on stream.  Batches of >= 65536
- * rays with dldv use the context's ray-order scratch (see the
- * "adjoint_sort" option; ordered across streams like the other users). */
+ * rays with dldv (see the "adjoint_sort" option) use scratch kept by the
+ * context and ordered across streams like its other users: 33 bytes per ray
+ * for the bins, allocated, after a device synchronisation, by the first call
+ * of each larger size.  Where that memory is not there, under capture before
+ * such a call, and for meshes above 1 048 320 triangles, rays are sorted in
+ * the ray-order scratch instead (16 bytes per ray and the sort's counts). */
 int xdg_hip_ray_distance_adjoint(xdg_hip_ctx* ctx, int64_t n, const double* org, const double* dir,
                                  const double* t, const int32_t* face, const double* dldt, int64_t nv,
                                  const double* verts, int64_t ntri, const int32_t* tris, double* dldv,

@@ -88,3 +88,42 @@ def test_binned_adjoint_extreme_weights(ctx, value):
     for part in (fin & big[:, None], fin & ~big[:, None]):
         scale = np.abs(ov[part]).max(initial=0.0)
         assert np.allclose(gv[part], ov[part], rtol=1e-12, atol=1e-12 * scale)
+
+
+def test_sorted_form_under_capture():
+    """Captured on a context without bins but with ray-order scratch of that
+    size: the sorted form, replayed between eager calls."""
+    from xdg_amd import capi
+    c = capi.Context(0)
+    m = G.perturbed_sphere(3, 10.0, 0.05)
+    n = 70000
+    org, dirs, w = P.ball_points(9, 0, n, 9.0), P.iso_dirs(9, 1, n), P.normals(9, 2, n)
+    verts, tris = dev(torch, m.verts), dev(torch, m.tris)
+    o, d, dw = dev(torch, org), dev(torch, dirs), dev(torch, w)
+    v9, f, s, fl = m.tree_arrays(1)
+    tree = c.build_surface_tree(v9.reshape(-1, 3), np.arange(3 * len(f), dtype=np.int32).reshape(-1, 3), f, s, fl,
+                                m.bump(1))
+    c.set_option("ray_order", 1)
+    t, _, face = c.ray_fire(tree, o, d, precision=capi.MIXED)
+    gv, go, gd = torch.zeros_like(verts), torch.empty_like(o), torch.empty_like(d)
+    ov, oo, od = O.adjoint(m.verts, m.tris, org, dirs, host(t), host(face), w)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gv.zero_()
+        c.ray_distance_adjoint(o, d, t, face, dw, verts, tris, gv, go, gd,
+                               stream=torch.cuda.current_stream().cuda_stream)
+    ev = torch.zeros_like(verts)
+    for k in range(4):
+        go.fill_(float(k))
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(host(go)), bits(oo)) and np.array_equal(bits(host(gd)), bits(od))
+        assert np.allclose(host(gv), ov, rtol=1e-12, atol=1e-12 * np.abs(ov).max())
+        c.ray_fire(tree, o, d, precision=capi.MIXED)  # eager work on the same scratch
+        if k:  # binned, in memory of its own
+            ev.zero_()
+            c.ray_distance_adjoint(o, d, t, face, dw, verts, tris, ev, go, gd)
+            assert np.allclose(host(ev), ov, rtol=1e-12, atol=1e-12 * np.abs(ov).max())
+        torch.cuda.synchronize()
+    c.close()

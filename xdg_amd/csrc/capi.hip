@@ -367,7 +367,8 @@ const RayOrderScratch& order_scratch(xdg_hip_ctx* c, int64_t n)
 }
 
 // the binned adjoint's memory for n rays (grown on demand, kept by the
-// context); null under capture when it would have to grow
+// context); null when it would have to grow under capture, or the device has
+// not that much left (the sorted form takes about half of it)
 void* adjoint_scratch(xdg_hip_ctx* c, int64_t n, hipStream_t s)
 {
   if (n > c->adj_cap) {
@@ -376,7 +377,13 @@ void* adjoint_scratch(xdg_hip_ctx* c, int64_t n, hipStream_t s)
     if (c->d_adj) XDG_HIP_CHECK(hipFree(c->d_adj));
     c->d_adj = nullptr;
     c->adj_cap = 0;
-    XDG_HIP_CHECK(hipMalloc(&c->d_adj, adjoint_bins_bytes(n)));
+    const hipError_t e = hipMalloc(&c->d_adj, adjoint_bins_bytes(n));
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      c->d_adj = nullptr;
+      return nullptr;
+    }
+    XDG_HIP_CHECK(e);
     c->adj_cap = n;
   }
   return c->d_adj;
