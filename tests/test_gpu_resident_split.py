@@ -76,8 +76,8 @@ def test_point_in_volume_split(setup, n, prec):
 
 @pytest.mark.parametrize("n", [1, 3, 65, 4097, 65537, 300001])
 def test_closest_split(setup, n):
-    """closest on a closed shell with points near and far, and at its centre
-    (nearly as far from every triangle: the wave finishes those together)."""
+    """closest on a closed shell with points near, far and (every 101st) close
+    to its centre, nearly as far from every triangle."""
     import pyoracle as O
     ctx, m, vols, trees, pts, dirs, tpr = setup
     p = host(pts)[:n].copy()

@@ -1323,7 +1323,7 @@ int xdg_hip_closest(xdg_hip_ctx* c, int32_t tree, int64_t n, const double* pts, 
     if (n == 0) return XDG_HIP_OK;
     require(pts && dist_out && face_out, "null array");
     ClosestArgs a{c->d_surf, (int32_t)c->surf.size(), tree, n, pts, dist_out, face_out};
-    launch_closest(a, cfg_for(c, t.dev.depth), t.dev.stack4, pick(c, stream));
+    launch_closest(a, cfg_for(c, t.dev.depth), t.dev, pick(c, stream));
     XDG_HIP_CHECK(hipGetLastError());
     return XDG_HIP_OK;
   });

@@ -262,8 +262,8 @@ struct ClosestArgs {
   double* dist;
   int32_t* face;
 };
-// stack4: the tree's BVH4 stack bound (c.stack holds the binary depth)
-void launch_closest(const ClosestArgs& a, const LaunchCfg& c, int stack4, hipStream_t s);
+// t: the tree's descriptor (c.stack holds the binary depth)
+void launch_closest(const ClosestArgs& a, const LaunchCfg& c, const xdgd::SurfTreeDev& t, hipStream_t s);
 
 // ---- batched particle random walk (transport.hip) -------------------------
 // Device-resident problem (arrays owned by the context's transport handle).

@@ -556,8 +556,8 @@ __device__ __forceinline__ double box_d2(const double* b, const D3& p)
 }
 
 // The triangles of one leaf against the best distance and face so far (ties:
-// the smaller face).
-__device__ __forceinline__ void closest_tri(const SurfTreeDev& T, int32_t first, int32_t cnt, const D3& p,
+// the smaller face).  reject: farther ones by their FP32 bound first.
+__device__ __forceinline__ void closest_tri(const SurfTreeDev& T, int32_t first, int32_t cnt, const D3& p, bool reject,
                                             double& best, int32_t& bface)
 {
   for (int32_t j = 0; j < cnt; ++j) {
@@ -566,7 +566,7 @@ __device__ __forceinline__ void closest_tri(const SurfTreeDev& T, int32_t first,
     const D3 v0 = d3(r->v[0], r->v[1], r->v[2]);
     const D3 v1 = d3(r->v[3], r->v[4], r->v[5]);
     const D3 v2 = d3(r->v[6], r->v[7], r->v[8]);
-    if (closest_beyond(v0, v1, v2, d3(pn[0], pn[1], pn[2]), p, f32_up(best * best))) continue;
+    if (reject && closest_beyond(v0, v1, v2, d3(pn[0], pn[1], pn[2]), p, f32_up(best * best))) continue;
     const D3 q = closest_on_triangle(v0, v1, v2, p);
     const D3 e = sub(q, p);
     const double dist = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
@@ -575,44 +575,6 @@ __device__ __forceinline__ void closest_tri(const SurfTreeDev& T, int32_t first,
       best = dist;
       bface = face;
     }
-  }
-}
-
-// Distance and face of one point by the binary tree's FP64 boxes: points
-// beyond the FP32 boxes' limit.
-__device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* stk, int stride, int cap, double& best,
-                                    int32_t& bface)
-{
-  int sp = 0;
-  int32_t node = T.root;
-  while (true) {
-    if (node >= 0) {
-      const NodeD nd = T.nodes_d[node];
-      double d0 = box_d2(nd.b0, p), d1 = box_d2(nd.b1, p);
-      double lim = best * best;
-      bool h0 = d0 <= lim, h1 = d1 <= lim;
-      int32_t c0 = nd.c0, c1 = nd.c1;
-      if (h0 && h1) {
-        if (d1 < d0) {
-          int32_t tmp = c0;
-          c0 = c1;
-          c1 = tmp;
-        }
-        if (sp < cap) stk[sp++ * stride] = c1;
-        node = c0;
-      } else if (h0) {
-        node = c0;
-      } else if (h1) {
-        node = c1;
-      } else {
-        if (sp == 0) break;
-        node = stk[--sp * stride];
-      }
-      continue;
-    }
-    closest_tri(T, leaf_first(node), leaf_count(node), p, best, bface);
-    if (sp == 0) break;
-    node = stk[--sp * stride];
   }
 }
 
@@ -643,6 +605,34 @@ __device__ __forceinline__ void node4_dist(const Node4F* nodes, int32_t node, co
   cswap(te[1], ch[1], te[2], ch[2]);
 }
 
+// The same in FP64 for a point beyond the FP32 boxes' limit, whose distances
+// to them FP32 does not tell apart: the dilated boxes as they are, and a
+// factor on the limit for the rounding of a distance far beyond the bump.
+// te holds what each distance adds to the least of the four.
+__device__ __forceinline__ void node4_dist_far(const Node4D* nodes, int32_t node, const D3& p, double best, float* te,
+                                               int32_t* ch)
+{
+  const auto nd = as_global(nodes + node);
+  const double lim = best * best * (1.0 + 0x1p-48);
+  double d[4], least = INFINITY;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const double ex = fmax(fmax(nd->lox[i] - p.x, p.x - nd->hix[i]), 0.0);
+    const double ey = fmax(fmax(nd->loy[i] - p.y, p.y - nd->hiy[i]), 0.0);
+    const double ez = fmax(fmax(nd->loz[i] - p.z, p.z - nd->hiz[i]), 0.0);
+    d[i] = ex * ex + ey * ey + ez * ez;
+    ch[i] = d[i] <= lim ? nd->child[i] : CHILD_EMPTY;
+    if (ch[i] != CHILD_EMPTY) least = fmin(least, d[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) te[i] = ch[i] != CHILD_EMPTY ? (float)(d[i] - least) : INFINITY;
+  cswap(te[0], ch[0], te[1], ch[1]);
+  cswap(te[2], ch[2], te[3], ch[3]);
+  cswap(te[0], ch[0], te[2], ch[2]);
+  cswap(te[1], ch[1], te[3], ch[3]);
+  cswap(te[1], ch[1], te[2], ch[2]);
+}
+
 // LDS of one wave of k_closest: up to 64 points and the queues they share.
 // A queue entry is a child code and a tag: the point's lane, and the upper
 // half of the entry's FP32 box distance (a lower bound).
@@ -659,7 +649,7 @@ struct ClosestLds {
   int32_t leaf[CLOSEST_LEAVES];
   uint32_t ltag[CLOSEST_LEAVES];
   uint32_t ntag[CLOSEST_NODES];
-  int32_t node[CLOSEST_NODES];  // last: also the stacks of closest_fp64
+  int32_t node[CLOSEST_NODES];
 };
 __device__ __forceinline__ uint32_t closest_tag(int owner, float d)
 {
@@ -701,6 +691,74 @@ __device__ __forceinline__ void closest_push(ClosestLds& L, int owner, const flo
   }
 }
 
+// The steps of one batch of points until both queues are empty.  FAR: some
+// of them (fars, by lane) are beyond the FP32 boxes' limit; without any, the
+// steps carry no FP64 boxes (which cost them 4 to 9 % of their time).
+template <bool FAR>
+__device__ __forceinline__ void closest_run(ClosestLds& L, const SurfTreeDev& T, unsigned long long fars, bool queued,
+                                            int reserve, int nn, int nl)
+{
+  const int lane = threadIdx.x;
+  while (nn + nl > 0) {
+    if (nl < 64 && nn > 0) {
+      const int m = nn + 3 * 64 + reserve <= CLOSEST_NODES ? (nn < 64 ? nn : 64) : 1;
+      float te[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+      int32_t ch[4] = {CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY};
+      int owner = 0;
+      if (lane < m) {
+        const int k = nn - 1 - lane;
+        const uint32_t tag = L.ntag[k];
+        owner = (int)(tag & 63u);
+        const float lim = L.lim[owner];
+        if (FAR && (fars >> owner & 1)) {
+          node4_dist_far(T.nodes4_d, L.node[k], d3(L.px[owner], L.py[owner], L.pz[owner]),
+                         __longlong_as_double((long long)L.best[owner]), te, ch);
+          te[0] = te[1] = te[2] = te[3] = 0.0f;  // entries of far points always live
+        } else if (closest_live(tag, lim)) {
+          node4_dist(T.nodes4_f, L.node[k], L.c[owner], lim, te, ch);
+        }
+      }
+      nn -= m;
+      wave_lds_sync();
+      closest_push(L, owner, te, ch, nn, nl);
+    } else {
+      const int m = nl < 64 ? nl : 64;
+      bool cand = false;
+      int owner = 0;
+      double b = INFTY, b0 = INFTY;
+      int32_t f = INT32_MAX;
+      if (lane < m) {
+        const int k = nl - 1 - lane;
+        const uint32_t tag = L.ltag[k];
+        owner = (int)(tag & 63u);
+        if (closest_live(tag, L.lim[owner])) {
+          b = b0 = __longlong_as_double((long long)L.best[owner]);
+          f = L.face[owner];
+          const int32_t f0 = f, code = L.leaf[k];
+          closest_tri(T, leaf_first(code), leaf_count(code), d3(L.px[owner], L.py[owner], L.pz[owner]),
+                      !FAR || !(fars >> owner & 1), b, f);
+          cand = b < b0 || f != f0;
+        }
+      }
+      nl -= m;
+      if (__ballot(cand)) {
+        // several lanes may hold one point's leaves: the least distance
+        // first, then the smallest face at that distance
+        const unsigned long long bits = (unsigned long long)__double_as_longlong(b);
+        if (cand) atomicMin(&L.best[owner], bits);
+        wave_lds_sync();
+        const bool win = cand && L.best[owner] == bits;
+        if (win && b < b0) L.face[owner] = INT32_MAX;
+        wave_lds_sync();
+        if (win) atomicMin(&L.face[owner], f);
+        wave_lds_sync();
+        if (queued) L.lim[lane] = closest_limit(__longlong_as_double((long long)L.best[lane]));
+      }
+    }
+    wave_lds_sync();
+  }
+}
+
 // closest over the BVH4, one wave per workgroup.  A wave holds up to 64
 // points and works on their descents together: node and leaf entries of all
 // points share two LDS queues, and each step takes up to 64 entries of one
@@ -712,13 +770,19 @@ __device__ __forceinline__ void closest_push(ClosestLds& L, int owner, const flo
 // Steps take nodes while fewer than 64 leaves wait, else leaves.  While the
 // node queue has no room for a full step's pushes (3 x 64 net) above
 // `reserve` entries (the BVH4's stack bound), nodes are taken one at a time:
-// depth first, at most that many more entries, so it cannot overflow.  cap
-// is the binary tree's depth, for the FP64 descents.
+// depth first, at most that many more entries, so it cannot overflow.
+//
+// lead: each lane first takes its own point's nearest child down to a leaf.
+// With that leaf's distance as limit the queues stay short; without one they
+// fill with every point's siblings of its first path, and in trees of 80 000
+// triangles run the node queue into its one-at-a-time mode (1 M points near
+// a sphere of 81 920 triangles 1.35 -> 0.49 ms, 100 003 of them 0.130 ->
+// 0.075, 4 000 0.061 -> 0.042).
 // 100 003 points in a ball around a sphere of 20 480 triangles: 7.4 -> 0.35 ms
 // (a descent per lane on these boxes, the last 16 points of a wave finished
 // by all its lanes: 0.73 ms).  Bound by the latency of the steps, two waves
 // per SIMD (19 KB of LDS each).
-__global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int cap, int reserve, int lanes_first)
+__global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int lanes_first, bool lead)
 {
   extern __shared__ __align__(16) unsigned char smem[];
   ClosestLds& L = *(ClosestLds*)smem;
@@ -733,84 +797,46 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int cap, int rese
     const unsigned long long first = lanes_first < 64 ? (1ull << lanes_first) - 1ull : ~0ull;
     const int64_t pi = w.take(first, a.n, lanes_first);
     const bool have = lane < lanes_first && pi < a.n;
-    bool queued = false;
+    const bool queued = have && T.n_prims > 0;
+    bool far = false;
     if (have) {
       const D3 p = d3(a.pts[3 * pi], a.pts[3 * pi + 1], a.pts[3 * pi + 2]);
+      const ClosestPointF c = closest_point(p, shrink);
+      far = !(fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z)) <= limit);
       double best = INFTY;
       int32_t bface = INT32_MAX;
-      if (T.n_prims > 0) {
-        if (fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z)) <= limit)
-          queued = true;
-        else
-          closest_fp64(T, p, L.node + lane, 64, cap, best, bface);
+      int32_t node = lead && queued ? T.root4 : CHILD_EMPTY;
+      float te[4];
+      int32_t ch[4];
+      while (node >= 0 && !far) {
+        node4_dist(T.nodes4_f, node, c, INFINITY, te, ch);
+        node = ch[0];
       }
+      while (node >= 0) {
+        node4_dist_far(T.nodes4_d, node, p, best, te, ch);
+        node = ch[0];
+      }
+      if (node != CHILD_EMPTY) closest_tri(T, leaf_first(node), leaf_count(node), p, false, best, bface);
       L.px[lane] = p.x;
       L.py[lane] = p.y;
       L.pz[lane] = p.z;
-      L.c[lane] = closest_point(p, shrink);
+      L.c[lane] = c;
       L.best[lane] = (unsigned long long)__double_as_longlong(best);
       L.face[lane] = bface;
-      L.lim[lane] = INFINITY;
+      L.lim[lane] = closest_limit(best);
     }
+    const unsigned long long fars = __ballot(far);
     int nn = 0, nl = 0;  // entries in the node and leaf queues
     {
       const float te[4] = {0.0f, INFINITY, INFINITY, INFINITY};
       const int32_t ch[4] = {queued ? T.root4 : CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY};
-      wave_lds_sync();  // every lane's closest_fp64 stack is done with
       closest_push(L, lane, te, ch, nn, nl);
     }
     wave_lds_sync();
-    while (nn + nl > 0) {
-      if (nl < 64 && nn > 0) {
-        const int m = nn + 3 * 64 + reserve <= CLOSEST_NODES ? (nn < 64 ? nn : 64) : 1;
-        float te[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
-        int32_t ch[4] = {CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY, CHILD_EMPTY};
-        int owner = 0;
-        if (lane < m) {
-          const int k = nn - 1 - lane;
-          const uint32_t tag = L.ntag[k];
-          owner = (int)(tag & 63u);
-          const float lim = L.lim[owner];
-          if (closest_live(tag, lim)) node4_dist(T.nodes4_f, L.node[k], L.c[owner], lim, te, ch);
-        }
-        nn -= m;
-        wave_lds_sync();
-        closest_push(L, owner, te, ch, nn, nl);
-      } else {
-        const int m = nl < 64 ? nl : 64;
-        bool cand = false;
-        int owner = 0;
-        double b = INFTY, b0 = INFTY;
-        int32_t f = INT32_MAX;
-        if (lane < m) {
-          const int k = nl - 1 - lane;
-          const uint32_t tag = L.ltag[k];
-          owner = (int)(tag & 63u);
-          if (closest_live(tag, L.lim[owner])) {
-            b = b0 = __longlong_as_double((long long)L.best[owner]);
-            f = L.face[owner];
-            const int32_t f0 = f, code = L.leaf[k];
-            closest_tri(T, leaf_first(code), leaf_count(code), d3(L.px[owner], L.py[owner], L.pz[owner]), b, f);
-            cand = b < b0 || f != f0;
-          }
-        }
-        nl -= m;
-        if (__ballot(cand)) {
-          // several lanes may hold one point's leaves: the least distance
-          // first, then the smallest face at that distance
-          const unsigned long long bits = (unsigned long long)__double_as_longlong(b);
-          if (cand) atomicMin(&L.best[owner], bits);
-          wave_lds_sync();
-          const bool win = cand && L.best[owner] == bits;
-          if (win && b < b0) L.face[owner] = INT32_MAX;
-          wave_lds_sync();
-          if (win) atomicMin(&L.face[owner], f);
-          wave_lds_sync();
-          if (queued) L.lim[lane] = closest_limit(__longlong_as_double((long long)L.best[lane]));
-        }
-      }
-      wave_lds_sync();
-    }
+    if (fars)
+      closest_run<true>(L, T, fars, queued, reserve, nn, nl);
+    else
+      closest_run<false>(L, T, fars, queued, reserve, nn, nl);
     if (have) {
       const int32_t f = L.face[lane];
       a.dist[pi] = f == INT32_MAX ? INFTY : __longlong_as_double((long long)L.best[lane]);
@@ -818,6 +844,60 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int cap, int rese
     }
     wave_lds_sync();
   }
+}
+
+// Distance and face of one point by the binary tree's FP64 boxes, one point
+// per lane: large batches on a tree of a few triangles, whose descents are
+// alike (launch_closest).
+__device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* stk, int stride, int cap, double& best,
+                                    int32_t& bface)
+{
+  int sp = 0;
+  int32_t node = T.root;
+  while (true) {
+    if (node >= 0) {
+      const NodeD nd = T.nodes_d[node];
+      double d0 = box_d2(nd.b0, p), d1 = box_d2(nd.b1, p);
+      double lim = best * best;
+      bool h0 = d0 <= lim, h1 = d1 <= lim;
+      int32_t c0 = nd.c0, c1 = nd.c1;
+      if (h0 && h1) {
+        if (d1 < d0) {
+          int32_t tmp = c0;
+          c0 = c1;
+          c1 = tmp;
+        }
+        if (sp < cap) stk[sp++ * stride] = c1;
+        node = c0;
+      } else if (h0) {
+        node = c0;
+      } else if (h1) {
+        node = c1;
+      } else {
+        if (sp == 0) break;
+        node = stk[--sp * stride];
+      }
+      continue;
+    }
+    closest_tri(T, leaf_first(node), leaf_count(node), p, false, best, bface);
+    if (sp == 0) break;
+    node = stk[--sp * stride];
+  }
+}
+
+__global__ void k_closest_lane(ClosestArgs a, int cap)
+{
+  extern __shared__ int32_t lds[];
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const SurfTreeDev& T = a.table[a.tree];
+  double best = INFTY;
+  int32_t bface = INT32_MAX;
+  if (T.n_prims > 0)
+    closest_fp64(T, d3(a.pts[3 * i], a.pts[3 * i + 1], a.pts[3 * i + 2]), lds + threadIdx.x, blockDim.x, cap, best,
+                 bface);
+  a.dist[i] = bface == INT32_MAX ? INFTY : best;
+  a.face[i] = bface == INT32_MAX ? ID_NONE : bface;
 }
 
 inline dim3 grid1(int64_t n, int blk) { return dim3((unsigned)((n + blk - 1) / blk)); }
@@ -1037,16 +1117,27 @@ void launch_occluded(const OccludedArgs& a, bool mixed, const LaunchCfg& c, hipS
   XDG_DISPATCH2(k_occluded, mixed, c.wide, grid1(a.n, c.block), dim3(c.block), lds_bytes(c), s, a, c.stack);
 }
 
-void launch_closest(const ClosestArgs& a, const LaunchCfg& c, int stack4, hipStream_t s)
+void launch_closest(const ClosestArgs& a, const LaunchCfg& c, const SurfTreeDev& t, hipStream_t s)
 {
   if (a.n <= 0) return;
-  const size_t sh = offsetof(ClosestLds, node) + sizeof(int32_t) * (size_t)std::max(CLOSEST_NODES, 64 * c.stack);
+  // 20 triangles, 1 M points (lane / queues): around the sphere 0.190 / 0.20
+  // ms, near it 0.135 / 0.18; 100 003: 0.062 / 0.046 and 0.047 / 0.045; 80
+  // triangles, 1 M around: 0.51 / 0.28
+  if (t.n_prims <= 32 && a.n >= 1 << 19) {
+    hipLaunchKernelGGL(k_closest_lane, grid1(a.n, c.block), dim3(c.block), lds_bytes(c), s, a, c.stack);
+    return;
+  }
+  const size_t sh = sizeof(ClosestLds);
   // spread over every resident wave: its lanes are busy however few points
   // it holds
   const int64_t waves = resident_grid(k_closest, 64, sh);
   const int lanes_first = (int)std::min<int64_t>(64, (a.n + waves - 1) / waves);
   const unsigned grid = (unsigned)std::min<int64_t>(waves, (a.n + lanes_first - 1) / lanes_first);
-  hipLaunchKernelGGL(k_closest, dim3(grid), dim3(64), sh, s, a, c.stack, stack4, lanes_first);
+  // the leading descent costs a few waves of a handful of points more than it
+  // saves in a tree of a few levels (80 triangles, 4 000 points: 32 us without
+  // it, 35 with; 320: 41 and 41; 80 triangles, 20 000 points: 42 and 38)
+  const bool lead = t.n_prims > 256 || lanes_first >= 8;
+  hipLaunchKernelGGL(k_closest, dim3(grid), dim3(64), sh, s, a, t.stack4, lanes_first, lead);
 }
 
 // ---- primitive evaluation (parity checks of the device geometry kernels) --
