@@ -200,7 +200,9 @@ def bench_ray_fire(args, ctx, torch, stream, sh):
     flops_ray = 40 * V + 9 * F + 23 * E + 26 * Cf + 29 * N
     achieved = bytes_ray * n / avg_m / 1e9
     fp64_tflops = flops_ray * n / avg_m / 1e12
-    # the BVH4 the kernel actually walks, and its divergence
+    # the BVH4 the kernel walks, and the divergence of one ray per lane on it
+    # (the timed resident grid refills lanes: its lane utilisation is in
+    # profiles/ray_fire_nested_spheres_sq_counters.md)
     s4 = ctx.ray_fire_stats(0, sub[0], sub[1], tree_per_ray=sub[2], precision=capi.MIXED)
     V4 = s4["nodes"] / s4["rays"]
     simd_node = s4["nodes"] / (64 * max(s4["wave_node_iters"], 1))

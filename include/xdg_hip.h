@@ -97,11 +97,11 @@ const char* xdg_hip_last_error(const xdg_hip_ctx* ctx);
 int xdg_hip_set_launch(xdg_hip_ctx* ctx, int block, int stack);
 int xdg_hip_get_launch(xdg_hip_ctx* ctx, int* block, int* stack);
 /* Traversal variant: wide != 0 uses the 4-wide tree (default), else the
- * binary tree it is collapsed from; defer != 0 (default) traces far-origin mixed ray_fire rays in
- * a separate FP64 pass; persistent selects resident-grid kernels whose
- * lanes claim new work from a counter as they finish (bit 0 plain
- * ray_fire, bit 1 mixed ray_fire, bit 2 find_volume; default 7).  Results
- * are identical either way. */
+ * binary tree it is collapsed from; defer != 0 (default) traces far-origin
+ * mixed ray_fire rays in a separate FP64 pass; persistent selects
+ * resident-grid kernels whose lanes take new work as they finish (bit 0
+ * plain ray_fire, bit 1 mixed ray_fire, bit 2 find_volume and
+ * point_in_volume; default 7).  Results are identical either way. */
 int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent);
 /* Tuning options by name (no counterpart in the reference; results are
  * identical for every setting):
@@ -125,8 +125,8 @@ int xdg_hip_set_traversal(xdg_hip_ctx* ctx, int wide, int defer, int persistent)
  *                 order (0).  Only speed differs, never results
  *   "refill"      persistent ray_fire: idle lanes a wave waits for before
  *                 it starts new rays (1..64, default 32)
- *   "fv_refill"   the same for the persistent find_volume (1..64; 0, the
- *                 default: 24)
+ *   "fv_refill"   the same for the persistent find_volume and
+ *                 point_in_volume (1..64; 0, the default: 24)
  *   "adjoint_sort" adjoint batches of >= 65536 rays with dldv: each face's
  *                 rays are summed before the vertex atomics (1, default), or
  *                 nine atomics per ray (0); dldv's FP64 summation order
@@ -248,8 +248,10 @@ int xdg_hip_ray_fire_noalloc(xdg_hip_ctx* ctx, int32_t tree, const int32_t* tree
                              const int32_t* excl, int k, int precision, double* t_out, int32_t* surf_out,
                              int32_t* face_out, void* stream);
 
-/* Instrumented xdg_hip_ray_fire (same traversal, no outputs) for roofline
- * accounting; synchronous.  counters (host, XDG_HIP_NUM_COUNTERS): rays, BVH
+/* Instrumented xdg_hip_ray_fire (one ray per lane, no outputs) for roofline
+ * accounting; synchronous.  The resident-grid kernels find the same hits but
+ * leave their node loop earlier and refill lanes, so their visits differ a
+ * little and their iterations per wave are not these.  counters (host, XDG_HIP_NUM_COUNTERS): rays, BVH
  * nodes visited, triangle tests, Pluecker edge tests, tests reaching the
  * distance computation, normal evaluations, hits, mixed-precision fallbacks
  * to FP64 boxes, node-loop iterations executed per wave (summed over waves),

@@ -1,6 +1,9 @@
-"""The transport start stage's FP32 volume prefilter never drops a volume that
-the FP64 slab test of the same dilated box reaches (arithmetic emulated on the
-CPU: boxes from 1e-3 to 1e6 away, near-axis and axis-parallel directions)."""
+"""The derivation of the transport start stage's FP32 volume prefilter, in
+numpy: with its extra slack it never drops a volume that the FP64 slab test of
+the same dilated box reaches, and without it it does (boxes from 1e-3 to 1e6
+away, near-axis and axis-parallel directions).  The kernel's own code, slots
+without hits and coordinates beyond FP32's range are checked by
+test_fp32_bounds.py."""
 import numpy as np
 
 F = np.float32

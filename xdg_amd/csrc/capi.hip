@@ -894,7 +894,7 @@ int xdg_hip_build_element_tree(xdg_hip_ctx* c, int64_t n_verts, const double* ve
     }
     dev_free_all(tmp);
     c->elem.push_back(std::move(t));
-      try {
+    try {
       sync_tables(c);
     } catch (...) {
       dev_free_all(c->elem.back().bufs);

@@ -164,8 +164,8 @@ struct LaunchCfg {
   int order = 0;  // ray_fire coherence ordering mode (0 = off)
   int spec = 1;   // ray_fire BVH4 node loop parks leaves until the wave holds one each
   int refill = 32; // persistent ray_fire: idle lanes of a wave needed before a refill
-  int fv_refill = 0;  // persistent find_volume: the same threshold (0: 24)
-  int adj_sort = 1;   // adjoint batches of >= 65536 rays: ordered by hit face, vertex sums per wave
+  int fv_refill = 0;  // persistent find_volume and point_in_volume: the same threshold (0: 24)
+  int adj_sort = 1;   // adjoint batches of >= 65536 rays: vertex terms summed per face before the atomics
   int mw_wave = 1;  // mesh walk: batched re-entry rays (wavefront) instead of inline ones
   int mw_refill = 32;  // mesh walk rounds on a resident grid, lanes claiming particles in batches of this many (0: off)
   int seg_order = 0;  // segment walks in Morton order of the start points

@@ -230,8 +230,9 @@ __global__ void k_ray_fire_pt_plain(RayFireArgs a, unsigned long long* next_ray,
   ray_fire_pt_body<false>(a, next_ray, c);
 }
 
-// Instrumented ray_fire: identical traversal, plus per-ray work counters
-// summed into counters[0..7] = rays, V, F, E, C, N, hits, mixed-fallbacks.
+// Instrumented ray_fire, one ray per lane: the traversal of k_ray_fire (the
+// resident grid leaves its node loop earlier and refills lanes, so its wave
+// iterations are fewer), plus per-ray work counters summed into counters[0..7] = rays, V, F, E, C, N, hits, mixed-fallbacks.
 template <bool MIXED, bool WIDE>
 __global__ void k_ray_fire_stats(RayFireArgs a, int cap, unsigned long long* counters, int spec)
 {
