@@ -1,5 +1,6 @@
-// CPU checks of xdg_amd/csrc/fp32_bounds.h, the conservative FP32 tests of
-// the kernels (host side of the same functions).  argv[1] names the check;
+// CPU checks of the kernels' conservative tests, which decide what gets the
+// full FP64 arithmetic (host side of the same functions): fp32_bounds.h, and
+// the early rejects of tet_contains.  argv[1] names the check;
 // prints "ok" or what failed.
 #include <cmath>
 #include <cstdio>
@@ -202,6 +203,55 @@ int start_boxes(double lo_exp, double hi_exp)
   return dropped || none || reached < n / 10;
 }
 
+// tet_contains without its early rejects
+bool contains(const D3& p, const D3& v0, const D3& v1, const D3& v2, const D3& v3)
+{
+  const D3 c0 = sub(v1, v0), c1 = sub(v2, v0), c2 = sub(v3, v0), r = sub(p, v0);
+  // rows of the adjugate: the cross products of the columns
+  const D3 b[3] = {cross(c1, c2), cross(c2, c0), cross(c0, c1)};
+  const double det = c0.x * b[0].x + c0.y * b[0].y + c0.z * b[0].z, hi = 1.0 + PLUCKER_ZERO_TOL;
+  double l[4], sum = 0.0;
+  for (int k = 0; k < 3; ++k) l[k] = b[k].x / det * r.x + b[k].y / det * r.y + b[k].z / det * r.z;
+  sum = l[0] + l[1] + l[2];
+  l[3] = 1.0 - sum;
+  for (double x : l)
+    if (x < -PLUCKER_ZERO_TOL || x > hi) return false;
+  return true;
+}
+
+// The early rejects change no answer: tets thin to flat, near to and far from
+// the origin, points on their faces, edges and vertices and a few ulps off
+// them, scales 1e-110 to 1e105.
+int containment()
+{
+  long wrong = 0;
+  for (int e = -110; e <= 105; e += 5) {
+    const double scale = std::pow(10.0, e);
+    long bad = 0, inside = 0;
+    for (int i = 0; i < 40000; ++i) {
+      const double thin = i % 3 ? 1.0 : std::pow(10.0, -17.0 * uni()), at = i % 2 ? 1.0 : 1e3;
+      const D3 o = rnd(at);
+      D3 v[4], p{0.0, 0.0, 0.0};
+      for (D3& q : v) q = D3{o.x + nrm(), o.y + nrm(), o.z + thin * nrm()};
+      double w[4], t = 0.0;
+      for (int k = 0; k < 4; ++k) t += w[k] = (i % 7 == k || (i % 7 < 2 && k == 3)) ? 0.0 : uni();
+      for (int k = 0; k < 4; ++k)
+        p = D3{p.x + w[k] / t * v[k].x, p.y + w[k] / t * v[k].y, p.z + w[k] / t * v[k].z};
+      if (i % 11 < 5) p.x *= 1.0 + (i % 11 - 2) * 0x1p-51;
+      if (i % 11 == 6) p = v[i % 4];
+      for (D3& q : v) q = D3{q.x * scale, q.y * scale, q.z * scale};
+      p = D3{p.x * scale, p.y * scale, p.z * scale};
+      const bool ref = contains(p, v[0], v[1], v[2], v[3]);
+      inside += ref;
+      bad += ref != tet_contains(p, v[0], v[1], v[2], v[3]);
+    }
+    if (bad) std::printf("scale 1e%d: %ld of 40000 answers differ\n", e, bad);
+    if (inside < 1000 || inside > 39000) std::printf("scale 1e%d: %ld of 40000 inside\n", e, inside);
+    wrong += bad;
+  }
+  return wrong != 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -212,6 +262,7 @@ int main(int argc, char** argv)
   if (argc == 2 && !std::strcmp(argv[1], "closest_boxes")) rc = closest_boxes();
   if (argc == 2 && !std::strcmp(argv[1], "start_boxes")) rc = start_boxes(-3.0, 6.0);
   if (argc == 2 && !std::strcmp(argv[1], "start_boxes_huge")) rc = start_boxes(6.0, 60.0);
+  if (argc == 2 && !std::strcmp(argv[1], "containment")) rc = containment();
   if (!rc) std::printf("ok\n");
   return rc;
 }

@@ -1,6 +1,7 @@
-"""The kernels' FP32 candidate tests (xdg_amd/csrc/fp32_bounds.h) on the CPU:
-tests/cpp/fp32_bounds_cpu.cpp compiles the functions themselves for the host
-and checks each against 64-bit or 80-bit arithmetic."""
+"""The kernels' conservative candidate tests (xdg_amd/csrc/fp32_bounds.h and
+tet_contains' early rejects) on the CPU: tests/cpp/fp32_bounds_cpu.cpp
+compiles the functions themselves for the host and checks each against 64-bit
+or 80-bit arithmetic."""
 import os
 import subprocess
 
@@ -18,7 +19,7 @@ def exe(tmp_path_factory):
     return str(out)
 
 
-@pytest.mark.parametrize("check", ["closest", "closest_thin", "closest_boxes", "start_boxes", "start_boxes_huge"])
+@pytest.mark.parametrize("check", ["closest", "closest_thin", "closest_boxes", "start_boxes", "start_boxes_huge", "containment"])
 def test_bound(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

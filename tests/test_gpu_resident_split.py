@@ -149,3 +149,60 @@ def test_element_records(setup, m, jitter):
     cnt, hsh = [host(x) for x in ctx.tally_segments(et, dev(torch, p0), dev(torch, p1))]
     rc, rh = om.segments(p0, p1)
     assert np.array_equal(cnt, rc) and np.array_equal(hsh.view(np.uint64), rh)
+
+
+def contains(p, v):
+    """The reference's containment test (tetrahedron_contain.cpp:11-43) of
+    points (n, 3) in tets (n, 4, 3), a zero determinant included."""
+    c = [v[:, k + 1] - v[:, 0] for k in range(3)]
+    r = p - v[:, 0]
+    cross = lambda a, b: np.stack([a[:, (i + 1) % 3] * b[:, (i + 2) % 3] - a[:, (i + 2) % 3] * b[:, (i + 1) % 3]
+                                   for i in range(3)], 1)
+    rows = [cross(c[1], c[2]), cross(c[2], c[0]), cross(c[0], c[1])]
+    det = c[0][:, 0] * rows[0][:, 0] + c[0][:, 1] * rows[0][:, 1] + c[0][:, 2] * rows[0][:, 2]
+    tol = 20.0 * 2.220446049250313e-16
+    with np.errstate(divide="ignore", invalid="ignore"):
+        lam = [b / det[:, None] * r for b in rows]
+        lam = [x[:, 0] + x[:, 1] + x[:, 2] for x in lam]
+        lam.append(1.0 - (lam[0] + lam[1] + lam[2]))
+        return ~np.any([(x < -tol) | (x > 1.0 + tol) for x in lam], axis=0)
+
+
+def test_flat_elements():
+    """Tets of zero volume among ordinary ones: with the reference's division
+    by a zero determinant they hold the points of their box for which no
+    coordinate comes out infinite."""
+    import pyoracle as O
+    from xdg_amd import capi
+    ctx = capi.Context(0)
+    ctx.set_option("leaf_size", 1)  # a flat element is asked about its own box only
+    rng = np.random.default_rng(93)
+    ref = G.kuhn_cube(5, 0.2, seed=4)
+    k = 200  # in lattice planes, whose coordinates are exact
+    lo = rng.integers(0, 8, (k, 3)) / 8.0
+    ax = rng.integers(0, 3, k)
+    flat = lo[:, None] + rng.integers(0, 3, (k, 4, 3)) / 16.0
+    flat[np.arange(k), :, ax] = lo[np.arange(k), ax, None]
+    tets = np.concatenate([len(ref.verts) + np.arange(4 * k, dtype=np.int32).reshape(k, 4), ref.tets])
+    verts = np.concatenate([ref.verts, flat.reshape(-1, 3)])
+    adj = np.full(tets.shape, -1, np.int32)
+    et = ctx.build_element_tree(verts, tets.astype(np.int32), adj, ref.face_order)
+    p = rng.random((20000, 3))
+    j = rng.integers(0, k, 10000)
+    w = rng.random((10000, 4, 1))
+    p[:10000] = (flat[j] * w).sum(1) / w.sum(1)
+    p[:3000] = flat[j[:3000], 0] + rng.random((3000, 1)) * (flat[j[:3000], 1] - flat[j[:3000], 0])
+    p[3000:4000] = flat[j[3000:4000], 2]
+    want = O.TetMesh(ref, with_ipc=False).find_element(p)
+    want = np.where(want >= 0, want + k, -1)
+    holds = 0
+    for e in range(k - 1, -1, -1):
+        # its dilated box (tetrahedron_contain.cpp:47-63): points of its plane
+        # up to rounding, no other point comes as near
+        in_box = ((p >= flat[e].min(0) - 1e-9) & (p <= flat[e].max(0) + 1e-9)).all(1)
+        c = in_box & contains(p, np.broadcast_to(flat[e], (len(p), 4, 3)))
+        holds += c.sum()
+        want = np.where(c, e, want)
+    assert holds > 500
+    assert np.array_equal(host(ctx.find_element(et, dev(torch, p))), want)
+    ctx.close()

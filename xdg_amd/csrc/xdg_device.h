@@ -303,8 +303,10 @@ __device__ inline D3 closest_on_triangle(const D3& v0, const D3& v1, const D3& v
 // n_k / det by a few units of 2^-53 of the terms' absolute sum m_k over
 // |det|, so n_k below -(tolerance + 2^-47 m_k) on det's scale puts lambda_k
 // below the tolerance (likewise lambda_0).  A zero or NaN det rejects
-// nothing here.
-__device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3& v1, const D3& v2, const D3& v3)
+// nothing here (the divisions make infinities and NaN of a flat tet, which
+// the comparisons below may accept), nor one so small that the tolerance on
+// its scale would round to zero.
+__host__ __device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3& v1, const D3& v2, const D3& v3)
 {
   const D3 c0 = sub(v1, v0);
   const D3 c1 = sub(v2, v0);
@@ -316,7 +318,8 @@ __device__ __forceinline__ bool tet_contains(const D3& p, const D3& v0, const D3
   const double det = c0.x * a0.x + c0.y * a1.x + c0.z * a2.x;
   const double hi = 1.0 + PLUCKER_ZERO_TOL;
   {
-    const double sg = det < 0.0 ? -1.0 : 1.0, ad = fabs(det), tol = 2.0 * PLUCKER_ZERO_TOL * ad;
+    const double sg = det < 0.0 ? -1.0 : 1.0, ad = fabs(det);
+    const double tol = ad > 0x1p-900 ? 2.0 * PLUCKER_ZERO_TOL * ad : (double)INFINITY;
     const double x1 = a0.x * r.x, y1 = a1.x * r.y, z1 = a2.x * r.z;
     const double x2 = a0.y * r.x, y2 = a1.y * r.y, z2 = a2.y * r.z;
     const double x3 = a0.z * r.x, y3 = a1.z * r.y, z3 = a2.z * r.z;
