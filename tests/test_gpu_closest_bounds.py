@@ -71,7 +71,7 @@ def test_closest_forms(ctx, ntri, n):
     v9 = v[t[rng.permutation(len(t))[:ntri]]].reshape(-1, 9)
     k = min(n, 4000)
     pts = P.ball_points(87, 0, k, 8.0)
-    pts[::7] *= 10.0 ** rng.uniform(3, 7, (len(pts[::7]), 1))
+    pts[::7] *= 10.0 ** rng.uniform(3, 15, (len(pts[::7]), 1))  # the last tie at every face
     pts[1::5] = v9[rng.integers(0, ntri, len(pts[1::5])), :3]
     pts[2::1001] = np.nan
     pts[3::1001, 1] = np.inf

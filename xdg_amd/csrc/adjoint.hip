@@ -385,8 +385,8 @@ size_t adjoint_bins_bytes(int64_t n)
 
 // Bound by the bytes of k_adj_rays: 116 in, 48 of ray gradients and 33 of
 // terms per ray.  4 M rays on 81 920 faces, whole call: one atomic set per
-// ray 1.6 ms, sorted by face (six radix passes) 1.02 ms, binned 0.42 ms
-// (rays 0.28, faces 0.07, count 0.03).
+// ray 1.6 ms, sorted by face (six radix passes) 1.02 ms, binned 0.40 ms
+// (rays 0.25, faces 0.07, count 0.03).
 void launch_adjoint_binned(const AdjointArgs& a, void* mem, hipStream_t s)
 {
   if (a.n <= 0) return;

@@ -341,10 +341,11 @@ __device__ __forceinline__ void next_element_dev(const ElemTreeDev& T, int32_t e
 
 // find_element on a resident grid: lanes whose point is located take the
 // next points of their wave's strided share together (no scratch, so
-// launches may overlap or be captured).  Bound by the latency of node and
-// element fetches outside L2 (1.57 M tets, 260 MB).  1 M points: binary tree,
-// one point per lane, nine divisions per candidate 0.78 ms; BVH4 with early
-// rejects 0.54 ms; refilled lanes 0.43 ms.
+// launches may overlap or be captured).  Bound by the node and
+// element lines it fetches past L2 (1.57 M tets, 260 MB: 2 KB per point, at
+// the 4.5 TB/s of a large copy).  1 M points: binary tree, one point per lane,
+// nine divisions per candidate 0.78 ms; BVH4 with early rejects 0.54 ms;
+// refilled lanes 0.44 ms.
 __global__ void k_find_element(FindElementArgs a, int lanes_first, int refill, int min_lanes)
 {
   extern __shared__ int32_t lds[];

@@ -232,7 +232,8 @@ __global__ void k_ray_fire_pt_plain(RayFireArgs a, unsigned long long* next_ray,
 
 // Instrumented ray_fire, one ray per lane: the traversal of k_ray_fire (the
 // resident grid leaves its node loop earlier and refills lanes, so its wave
-// iterations are fewer), plus per-ray work counters summed into counters[0..7] = rays, V, F, E, C, N, hits, mixed-fallbacks.
+// iterations are fewer), plus per-ray work counters summed into
+// counters[0..7] = rays, V, F, E, C, N, hits, mixed-fallbacks.
 template <bool MIXED, bool WIDE>
 __global__ void k_ray_fire_stats(RayFireArgs a, int cap, unsigned long long* counters, int spec)
 {
@@ -849,7 +850,7 @@ __global__ __launch_bounds__(64) void k_closest(ClosestArgs a, int reserve, int 
 
 // Distance and face of one point by the binary tree's FP64 boxes, one point
 // per lane: large batches on a tree of a few triangles, whose descents are
-// alike (launch_closest).
+// alike (launch_closest).  The limit's factor is node4_dist_far's.
 __device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* stk, int stride, int cap, double& best,
                                     int32_t& bface)
 {
@@ -859,7 +860,7 @@ __device__ inline void closest_fp64(const SurfTreeDev& T, const D3& p, int32_t* 
     if (node >= 0) {
       const NodeD nd = T.nodes_d[node];
       double d0 = box_d2(nd.b0, p), d1 = box_d2(nd.b1, p);
-      double lim = best * best;
+      double lim = best * best * (1.0 + 0x1p-48);
       bool h0 = d0 <= lim, h1 = d1 <= lim;
       int32_t c0 = nd.c0, c1 = nd.c1;
       if (h0 && h1) {
